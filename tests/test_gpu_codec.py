@@ -179,3 +179,29 @@ def test_decode_batch_records_layout(amd):
         single = amd.decode(rd, bits, k, n, codebook=1, layout=amd.LAYOUT_RECORDS)
         torch.cuda.synchronize()
         assert torch.equal(out, single), (bits, k, n)
+
+
+@pytest.mark.parametrize("bits,cb", [(b, c) for b in range(1, 9) for c in range(3) if (b + c) % 2 == 0])
+@pytest.mark.parametrize("records", [False, True])
+def test_reconstruct_wave_layout(amd, oracle, bits, cb, records):
+    """Every rate, both layouts, a column slice, an output at an odd 16-bit address, and blocks of
+    equal weights (their H128 cancels to exact zeros, whose sign counts): the same bits."""
+    import torch
+    k, n, first, count = 256, 384, 128, 256
+    p = synth.packed_tiles(900 + bits, k, n, bits)
+    p.reshape(k // 16, n // 16, -1)[:, 8:16] = 0  # one column group of all-zero states
+    su, sv = synth.layer_scales(900 + bits, k, n)
+    want = oracle.reconstruct(p, su, sv, k, n, bits, cb)[:, first: first + count]
+    print(f"  reconstruct bits={bits} cb={cb} records={records}", flush=True)
+    raw = torch.zeros(k * count + 8, dtype=torch.int16, device="cuda")
+    for shift in (0, 1):  # 16-byte aligned, and 2 bytes past that
+        out = raw[shift: shift + k * count].view(k, count)
+        if records:
+            src, su_t, sv_t = dev(synth.pack_records(p, su, sv, bits).view(np.uint8)), None, None
+            layout = amd.LAYOUT_RECORDS
+        else:
+            src, su_t, sv_t = dev(p), dev(su.view(np.uint16)), dev(sv.view(np.uint16))
+            layout = amd.LAYOUT_UPSTREAM_TILES
+        got = amd.reconstruct(src, bits, k, n, su=su_t, sv=sv_t, codebook=cb, layout=layout, first=first, count=count,
+                              out=out)
+        assert np.array_equal(host_u16(got), want.view(np.uint16)), (bits, cb, shift)

@@ -11,6 +11,8 @@
 
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "exl3_kernel_common.hpp"
 
 namespace exl3k {
@@ -250,75 +252,172 @@ hipError_t launch_decode(const void *src, int rl, int bits, int cb, size_t k, si
 }
 
 // ============================================================== reconstruct
-// One workgroup per 128x128 block: decode into LDS (fp32), H128 along each row
-// (over n), then along each column (over k), then fp16((w * su) * sv) -- the
-// operation order of src/exl3_codec.cpp:184-202, so the result is bit-exact.
+// A wave holds one tile row (16 rows x 128 columns, 8 tiles) of a 128-column
+// block, decoded a chunk per lane (decode_chunk): lane l, with b =
+// h128_lane_block(l % 16), has chunk j = b % 8 of tile tc = b / 8 + 2 (l / 16),
+// that is columns 16 tc + j and 16 tc + j + 8, all 16 rows.  Column bits 0, 1, 2, 4
+// (strides 1, 2, 4, 16) are then lane bits one DPP read apart (dpp_block_stage8),
+// bit 3 is the register, bits 5 and 6 are lane bits 4 and 5.  frag[f] holds rows
+// 8 (f % 2) .. + 7 of column 16 tc + j + 8 (f / 2), two rows per word.
 template <int K, int CB>
-__global__ __launch_bounds__(256) void reconstruct_kernel(const uint8_t *__restrict__ src, int records_layout,
+__device__ __forceinline__ void decode_tile_row(const uint8_t *__restrict__ src, int records_layout, size_t k,
+                                                size_t n, size_t rk, size_t cn0, int lane, u4 (&frag)[4]) {
+    const int b = h128_lane_block(lane & 15), j = b & 7, tc = (b >> 3) + 2 * (lane >> 4);
+    const uint32_t *tile = tile_ptr<K>(src, records_layout, k, n, rk, cn0 + tc);
+    uint32_t w[K];
+    load_chunk<K>((const uint8_t *)(tile + j * K), w);
+    // the previous chunk of the tile (cyclic): the lane holding block (j + 7) % 8
+    const int prev_lane = (lane & 48) | h128_lane_block((b & 8) | ((j + 7) & 7));
+    const uint32_t prev = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * prev_lane, (int)w[K - 1]);
+    decode_chunk<K, CB>(w, prev, frag);
+}
+
+// One workgroup of 8 waves per 128x128 block, wave tr its tile row tr.  H128 along
+// n stays in the wave: strides 1, 2, 4 and 16 are DPP fmacs, 8 is between registers,
+// and 32 and 64 exchange a lane bit with the register bit (permlane swaps), after
+// which the butterfly is between registers too.  H128 along k does strides 1..8 in
+// registers (a lane has all 16 rows of its columns), goes through LDS once, and does
+// 16..64 between the eight values a thread reads back (4 columns of row r of every
+// tile row).  Every sum has the operands and the stage order of
+// src/exl3_codec.cpp:184-202, then fp16((w * su) * sv): bit-exact.  The DPP stages
+// hold sgn times the value (round to nearest is sign-symmetric); the sign goes with
+// the 1/sqrt(128) scale as fma(v, +-scale, +0), whose +0 turns a negated exact zero
+// into the +0 that the plain butterflies give (no sum of theirs is -0: no codebook
+// value is, and x - x is +0).
+// Bound: VALU (about 30 per weight, ten of them the decode and its conversion) and
+// HBM: k = 2048, n = 6144, 4 bits 106.6 -> 10.9 us (31 MB: 2.9 TB/s), against one
+// thread per row, then per column, walking the block through LDS (two of four waves
+// idle, 2 x 7 x 64 dependent LDS steps).
+template <int K, int CB>
+__global__ __launch_bounds__(512) void reconstruct_kernel(const uint8_t *__restrict__ src, int records_layout,
                                                           const uint16_t *__restrict__ su,
                                                           const uint16_t *__restrict__ sv, size_t k, size_t n,
                                                           size_t first_column, size_t count,
                                                           uint16_t *__restrict__ out) {
-    constexpr int P = 129;
-    __shared__ float blk[128 * P];
-    const int tid = threadIdx.x;
+    constexpr float kScale = 0.08838834764831844055f;
+    __shared__ __attribute__((aligned(16))) float blk[8 * 16 * 128];  // [tile row][row][column]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int tr = __builtin_amdgcn_readfirstlane(tid >> 6);
     const size_t bc = blockIdx.x, brk = blockIdx.y;  // column block (within the slice), row block
-    const size_t cn0 = first_column / 16 + bc * 8, rk0 = brk * 8;
-#pragma unroll 1
-    for (int i = 0; i < 4; ++i) {
-        const int run = tid + 256 * i;
-        const int tile = run >> 4, rc = run & 15;
-        const int c = rc & 7, h = rc >> 3, tr = tile >> 3, tc = tile & 7;
-        const uint32_t *tp = tile_ptr<K>(src, records_layout, k, n, rk0 + tr, cn0 + tc);
-        uint32_t w[RunGeo<K>::NW];
-        load_run_words<K>(tp, c, h, w);
-        u4 a1, a2;
-        decode_run<K, CB>(w, a1, a2);
-        const uint32_t p1[4] = {a1.x, a1.y, a1.z, a1.w}, p2[4] = {a2.x, a2.y, a2.z, a2.w};
+    const size_t gcol0 = first_column + bc * 128;    // absolute column of this block
+    u4 frag[4];
+    decode_tile_row<K, CB>(src, records_layout, k, n, brk * 8 + tr, gcol0 / 16, lane, frag);
+    const int b = h128_lane_block(lane & 15);
+    float v[4][8];  // [f][row of the half]
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r0 = tr * 16 + run_slot_row(h, 2 * v), r1 = tr * 16 + run_slot_row(h, 2 * v + 1);
-            const int cc = tc * 16 + c;
-            blk[r0 * P + cc] = half_bits_to_float((uint16_t)(p1[v] & 0xffffu));
-            blk[r1 * P + cc] = half_bits_to_float((uint16_t)(p1[v] >> 16));
-            blk[r0 * P + cc + 8] = half_bits_to_float((uint16_t)(p2[v] & 0xffffu));
-            blk[r1 * P + cc + 8] = half_bits_to_float((uint16_t)(p2[v] >> 16));
+    for (int f = 0; f < 4; ++f) {
+        const uint32_t w[4] = {frag[f].x, frag[f].y, frag[f].z, frag[f].w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[f][i] = half_bits_to_float((uint16_t)(w[i >> 1] >> (16 * (i & 1))));
+    }
+    auto lane_stage = [&](auto sc) {
+        constexpr int S = decltype(sc)::value;
+        const float sgn = (b & S) ? -1.f : 1.f;
+#pragma unroll
+        for (int f = 0; f < 4; ++f) dpp_block_stage8<S>(v[f], sgn);
+    };
+    auto register_stage = [&]() {  // between column halves f and f + 2
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float lo = v[f][i], hi = v[f + 2][i];
+                v[f][i] = lo + hi;
+                v[f + 2][i] = lo - hi;
+            }
+    };
+    lane_stage(std::integral_constant<int, 1>{});
+    lane_stage(std::integral_constant<int, 2>{});
+    lane_stage(std::integral_constant<int, 4>{});
+    register_stage();                              // stride 8
+    lane_stage(std::integral_constant<int, 8>{});  // block bit 3: stride 16
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {  // strides 32 and 64: the register bit trades places with lane bit 4, then 5
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int x = __float_as_int(v[f][i]), y = __float_as_int(v[f + 2][i]);
+                const auto r = st == 0 ? __builtin_amdgcn_permlane16_swap(x, y, false, false)
+                                       : __builtin_amdgcn_permlane32_swap(x, y, false, false);
+                v[f][i] = __int_as_float(r[0]);
+                v[f + 2][i] = __int_as_float(r[1]);
+            }
+        register_stage();
+    }
+    const float scale = (__builtin_popcount(b) & 1) ? -kScale : kScale;
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[f][i] = __builtin_fmaf(v[f][i], scale, 0.f);
+    // H128 along k, strides 1, 2, 4 (rows of a half) and 8 (halves)
+#pragma unroll
+    for (int st = 1; st < 8; st <<= 1)
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (!(i & st)) {
+                    const float lo = v[f][i], hi = v[f][i | st];
+                    v[f][i] = lo + hi;
+                    v[f][i | st] = lo - hi;
+                }
+#pragma unroll
+    for (int f = 0; f < 4; f += 2)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float lo = v[f][i], hi = v[f + 1][i];
+            v[f][i] = lo + hi;
+            v[f + 1][i] = lo - hi;
         }
-    }
-    __syncthreads();
-    // H128 along n for each row, one thread per row, stage order of the reference
-    if (tid < 128) {
-        float *v = blk + tid * P;
-        for (int step = 1; step < 128; step <<= 1)
-            for (int b = 0; b < 64; ++b) {
-                const int i = ((b & ~(step - 1)) << 1) | (b & (step - 1));
-                const float a = v[i], c2 = v[i + step];
-                v[i] = a + c2;
-                v[i + step] = a - c2;
-            }
-        for (int i = 0; i < 128; ++i) v[i] *= 0.08838834764831844055f;
-    }
-    __syncthreads();
-    if (tid < 128) {
-        float *v = blk + tid;
-        for (int step = 1; step < 128; step <<= 1)
-            for (int b = 0; b < 64; ++b) {
-                const int i = ((b & ~(step - 1)) << 1) | (b & (step - 1));
-                const float a = v[i * P], c2 = v[(i + step) * P];
-                v[i * P] = a + c2;
-                v[(i + step) * P] = a - c2;
-            }
-        for (int i = 0; i < 128; ++i) v[i * P] *= 0.08838834764831844055f;
-    }
-    __syncthreads();
-    const size_t gcol0 = first_column + bc * 128;  // absolute column of this block
+    // this lane's column (+ 64 for f >= 2): after the swaps lane bit 4 is column bit 3, lane
+    // bit 5 column bit 5 and the register column bit 6; a wave writes 64 columns of one row
+    const int col = (b & 7) | ((lane >> 4) & 1) << 3 | (b >> 3) << 4 | (lane >> 5) << 5;
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) blk[(tr * 16 + 8 * (f & 1) + i) * 128 + col + 64 * (f >> 1)] = v[f][i];
+    // the scales this thread's outputs need: 4 columns, 8 rows
+    const int r = tid >> 5, c4 = (tid & 31) * 4;
     const uint8_t *rec = records_layout ? src + ((gcol0 >> 7) * (k >> 7) + brk) * group_bytes(K) : nullptr;
     const uint16_t *su_b = records_layout ? (const uint16_t *)(rec + 2048 * K) : su + brk * 128;
     const uint16_t *sv_b = records_layout ? (const uint16_t *)(rec + 2048 * K + 256) : sv + gcol0;
-    for (int e = tid; e < 128 * 128; e += 256) {
-        const int row = e >> 7, col = e & 127;
-        const float scaled = mul_rn_f32(blk[row * P + col], half_bits_to_float(su_b[row]));
-        out[(brk * 128 + row) * count + bc * 128 + col] = float_to_half_bits(mul_rn_f32(scaled, half_bits_to_float(sv_b[col])));
+    float suv[8], svv[4];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) suv[t] = half_bits_to_float(su_b[16 * t + r]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) svv[c] = half_bits_to_float(sv_b[c4 + c]);
+    __syncthreads();
+    float u[8][4];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const f4 q = *(const f4 *)(blk + (t * 16 + r) * 128 + c4);
+        u[t][0] = q.x;
+        u[t][1] = q.y;
+        u[t][2] = q.z;
+        u[t][3] = q.w;
+    }
+#pragma unroll
+    for (int st = 1; st < 8; st <<= 1)  // strides 16, 32, 64
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+            if (!(t & st))
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float lo = u[t][c], hi = u[t | st][c];
+                    u[t][c] = lo + hi;
+                    u[t | st][c] = lo - hi;
+                }
+    // out is only 2-byte aligned by contract: the hardware takes the 8-byte stores at any alignment
+    typedef uint32_t u2_any __attribute__((ext_vector_type(2), aligned(2)));
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        uint32_t h[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            h[c] = float_to_half_bits(mul_rn_f32(mul_rn_f32(mul_rn_f32(u[t][c], kScale), suv[t]), svv[c]));
+        const u2_any o = {h[0] | h[1] << 16, h[2] | h[3] << 16};
+        __builtin_nontemporal_store(o, (u2_any *)(out + (brk * 128 + 16 * t + r) * count + bc * 128 + c4));
     }
 }
 
@@ -326,7 +425,7 @@ template <int K>
 static hipError_t launch_reconstruct_k(const void *src, int rl, const uint16_t *su, const uint16_t *sv, int cb,
                                        size_t k, size_t n, size_t first, size_t count, uint16_t *out,
                                        hipStream_t stream) {
-    const dim3 grid((unsigned)(count / 128), (unsigned)(k / 128)), block(256);
+    const dim3 grid((unsigned)(count / 128), (unsigned)(k / 128)), block(512);
     const uint8_t *s = (const uint8_t *)src;
     switch (cb) {
     case 0: reconstruct_kernel<K, 0><<<grid, block, 0, stream>>>(s, rl, su, sv, k, n, first, count, out); break;
