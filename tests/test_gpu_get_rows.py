@@ -86,3 +86,26 @@ def test_get_rows_strides_bad_ids_and_empty(amd, oracle):
     assert empty.shape == (0, k)
     L = amd.lib()
     assert L.exl3_hip_get_rows(None, 4, 2, 128, 128, None, 1, None, 0, 128, None, None) == 1
+
+
+@pytest.mark.parametrize("count", [2, 9, 511, 512, 513, 1100])
+@pytest.mark.parametrize("bits,cb,k,n", [(6, 2, 256, 384), (3, 0, 128, 1280), (5, 1, 128, 640)])
+def test_get_rows_shared_column_groups(amd, oracle, count, bits, cb, k, n):
+    """Many ids per column group (more than one workgroup serves at once, windows of ids cut
+    between them), repeated and out-of-range ids among them, every column of the group, and a
+    column group of equal weights (exact zeros): every row as the oracle gives it."""
+    rng = np.random.default_rng(count * 8 + bits)
+    p = synth.packed_tiles(70 + bits, k, n, bits)
+    p.reshape(k // 16, n // 16, -1)[:, 8:16] = 0
+    su, sv = synth.layer_scales(70 + bits, k, n)
+    rec_h = synth.pack_records(p, su, sv, bits).view(np.uint8)
+    ids = rng.integers(0, n, count).astype(np.int32)
+    ids[: min(count, 130)] = np.arange(min(count, 130))  # all columns of one group
+    bad = rng.integers(1, count, max(1, count // 50))
+    ids[bad] = np.where(bad % 2 == 0, n, -1)
+    print(f"  get_rows shared {k}x{n} bits={bits} cb={cb} count={count}", flush=True)
+    got = amd.get_rows(dev(rec_h), bits, k, n, ids_tensor(ids), codebook=cb).cpu().numpy()
+    ok = (ids >= 0) & (ids < n)
+    want = oracle.get_rows(rec_h, bits, cb, k, n, ids[ok])
+    assert np.array_equal(got[ok].view(np.uint32), want.view(np.uint32))
+    assert np.all(got[~ok].view(np.uint32) == 0x7FC00000)

@@ -259,15 +259,17 @@ hipError_t launch_decode(const void *src, int rl, int bits, int cb, size_t k, si
 // (strides 1, 2, 4, 16) are then lane bits one DPP read apart (dpp_block_stage8),
 // bit 3 is the register, bits 5 and 6 are lane bits 4 and 5.  frag[f] holds rows
 // 8 (f % 2) .. + 7 of column 16 tc + j + 8 (f / 2), two rows per word.
+template <int K>
+__device__ __forceinline__ void load_tile_row(const uint8_t *__restrict__ src, int records_layout, size_t k, size_t n,
+                                              size_t rk, size_t cn0, int lane, uint32_t (&w)[K]) {
+    const int b = h128_lane_block(lane & 15), tc = (b >> 3) + 2 * (lane >> 4);
+    load_chunk<K>((const uint8_t *)(tile_ptr<K>(src, records_layout, k, n, rk, cn0 + tc) + (b & 7) * K), w);
+}
 template <int K, int CB>
-__device__ __forceinline__ void decode_tile_row(const uint8_t *__restrict__ src, int records_layout, size_t k,
-                                                size_t n, size_t rk, size_t cn0, int lane, u4 (&frag)[4]) {
-    const int b = h128_lane_block(lane & 15), j = b & 7, tc = (b >> 3) + 2 * (lane >> 4);
-    const uint32_t *tile = tile_ptr<K>(src, records_layout, k, n, rk, cn0 + tc);
-    uint32_t w[K];
-    load_chunk<K>((const uint8_t *)(tile + j * K), w);
+__device__ __forceinline__ void decode_tile_row(const uint32_t (&w)[K], int lane, u4 (&frag)[4]) {
+    const int b = h128_lane_block(lane & 15);
     // the previous chunk of the tile (cyclic): the lane holding block (j + 7) % 8
-    const int prev_lane = (lane & 48) | h128_lane_block((b & 8) | ((j + 7) & 7));
+    const int prev_lane = (lane & 48) | h128_lane_block((b & 8) | ((b + 7) & 7));
     const uint32_t prev = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * prev_lane, (int)w[K - 1]);
     decode_chunk<K, CB>(w, prev, frag);
 }
@@ -301,14 +303,16 @@ __global__ __launch_bounds__(512) void reconstruct_kernel(const uint8_t *__restr
     const size_t bc = blockIdx.x, brk = blockIdx.y;  // column block (within the slice), row block
     const size_t gcol0 = first_column + bc * 128;    // absolute column of this block
     u4 frag[4];
-    decode_tile_row<K, CB>(src, records_layout, k, n, brk * 8 + tr, gcol0 / 16, lane, frag);
+    uint32_t w[K];
+    load_tile_row<K>(src, records_layout, k, n, brk * 8 + tr, gcol0 / 16, lane, w);
+    decode_tile_row<K, CB>(w, lane, frag);
     const int b = h128_lane_block(lane & 15);
     float v[4][8];  // [f][row of the half]
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
-        const uint32_t w[4] = {frag[f].x, frag[f].y, frag[f].z, frag[f].w};
+        const uint32_t p[4] = {frag[f].x, frag[f].y, frag[f].z, frag[f].w};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[f][i] = half_bits_to_float((uint16_t)(w[i >> 1] >> (16 * (i & 1))));
+        for (int i = 0; i < 8; ++i) v[f][i] = half_bits_to_float((uint16_t)(p[i >> 1] >> (16 * (i & 1))));
     }
     auto lane_stage = [&](auto sc) {
         constexpr int S = decltype(sc)::value;
@@ -450,27 +454,68 @@ hipError_t launch_reconstruct(const void *src, int rl, const uint16_t *su, const
 }
 
 // ============================================================== get_rows
-// GET_ROWS on records (src/exl3-ggml.cpp:19-49).  Workgroup (r, kb) writes
-// out[r][128 kb .. +127] = column c = ids[r] % 128 of the original-basis
-// reconstruct of record (ids[r] / 128, kb) as a 128x128 matrix, fp16-rounded
-// (then widened for F32 output): decode into LDS (fp32), the H128 of each row
-// over n restricted to the operations output c depends on (the same
-// butterflies, in the same order, as the full transform: bit-exact), then the
-// full H128 of that column over k and fp16((w * su) * sv) as exl3::reconstruct.
+// GET_ROWS on records (src/exl3-ggml.cpp:19-49): out[r][128 kb .. +127] = column
+// c = ids[r] % 128 of the original-basis reconstruct of record (ids[r] / 128, kb) as
+// a 128x128 matrix, fp16-rounded (then widened for F32 output).  Workgroup (r, kb)
+// decodes that record once, wave tr its tile row tr (decode_tile_row), and serves up
+// to kGetRowsShare ids with it: the ids of r's window (kGetRowsWindow ids from a
+// multiple of it) with the same column group are numbered in order, the workgroup
+// whose own number is a multiple of kGetRowsShare takes its and the next ones, the
+// others end.  512 ids of a 151,936-row vocabulary lie in about 416 column groups, a
+// prompt's repeated tokens in fewer.
+// Per id the H128 over n is restricted to the operations output c depends on (the
+// same butterflies in the same order: bit-exact): a stage of stride 2^s keeps
+// lo + hi, or lo - hi where bit s of c is set.  Strides 1, 2, 4 and 16 pair lanes, and
+// each halves a lane's rows: of two rows A and B the lower lane keeps A's result and
+// the upper one B's, so a stage costs two selects, one DPP move and one fma per pair.
+// The H128 of the column over k, then fp16((w * su) * sv), are exl3::reconstruct's.
+// A stage computes hi' + (+-1) own; where the difference is wanted the lower lane
+// holds its negative, and the sign goes with the 1/sqrt(128) scale as
+// fma(v, +-scale, +0), as in reconstruct_kernel.
 // An id outside [0, n) writes a NaN row and sets *bad_ids (if given) to 1.
+// Bound: VALU (about 7 per weight, four of them the decode, and 150 per wave around
+// it) and the chain ids -> words -> counting, hidden only by the four workgroups of a
+// CU.  512 ids of a k = 2048, n = 151,936, 6-bit table: 80.5 -> 39.1 us, against a
+// decode into LDS per id and one thread per row for the H128 over n.  With the ids
+// fastest in the grid instead of the records 44.3 us; without the shared decode about
+// a fifth more records; two records per workgroup 48.4 us (80 VGPRs: three workgroups
+// per CU).
+constexpr int kGetRowsThreads = 512;
+constexpr int kGetRowsWindow = kGetRowsThreads;  // one id per thread
+constexpr int kGetRowsShare = 8;                 // ids per decoded record: one per wave at the end
+
+// One lane-pair stage of two values A, B (rows kept by the lower and the upper lane
+// of the pair over block bit S): hi' + al own.  up is all ones on the upper lane: the
+// selects are v_bfi_b32, where a select on vcc would be v_cndmask_b32 in its short
+// form, which takes 18 cycles a wave here (the others 4).
+__device__ __forceinline__ uint32_t pick(uint32_t up, uint32_t a, uint32_t b) { return (up & b) | (~up & a); }
+template <int S>
+__device__ __forceinline__ float fold_pair(float a, float b, uint32_t up, float al) {
+    const uint32_t ai = __float_as_uint(a), bi = __float_as_uint(b);
+    const float own = __uint_as_float(pick(up, ai, bi)), send = __uint_as_float(pick(up, bi, ai));
+    return __builtin_fmaf(own, al, dpp_block_xor<S>(send));
+}
+
 template <int K, int CB>
-__global__ __launch_bounds__(256) void get_rows_kernel(const uint8_t *__restrict__ records, size_t k, size_t n,
-                                                       const int32_t *__restrict__ ids, size_t ids_stride,
-                                                       void *__restrict__ out, int out_f16, size_t out_stride,
-                                                       int *__restrict__ bad_ids) {
-    constexpr int P = 129;
-    __shared__ float blk[128 * P];
-    __shared__ float colv[128];
-    const int tid = threadIdx.x;
-    const size_t r = blockIdx.x, kb = blockIdx.y;
+__global__ __launch_bounds__(kGetRowsThreads) __attribute__((amdgpu_waves_per_eu(8))) void get_rows_kernel(
+    const uint8_t *__restrict__ records, size_t k, size_t n, const int32_t *__restrict__ ids, size_t ids_stride,
+    size_t count, void *__restrict__ out, int out_f16, size_t out_stride, int *__restrict__ bad_ids) {
+    constexpr float kScale = 0.08838834764831844055f;
+    constexpr int W = kGetRowsThreads / 64;
+    __shared__ float colv[kGetRowsShare][128];
+    __shared__ int matches[W];
+    __shared__ int member_row[kGetRowsShare], member_col[kGetRowsShare];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // records fastest: the workgroups in flight read whole column groups, each one contiguous
+    const size_t r = blockIdx.y + (size_t)gridDim.y * blockIdx.z, kb = blockIdx.x;
+    if (r >= count) return;
+    const size_t w0 = r - r % kGetRowsWindow;  // r's window of ids, one per thread
+    const int self = (int)(r - w0);
     const int32_t id = ids[r * ids_stride];
-    const size_t o = r * out_stride + kb * 128;
+    const int32_t other = ids[(w0 + tid < count ? w0 + tid : r) * ids_stride];
     if (id < 0 || (size_t)id >= n) {
+        const size_t o = r * out_stride + kb * 128;
         if (tid < 128) {
             if (out_f16) ((uint16_t *)out)[o + tid] = 0x7e00u;
             else ((uint32_t *)out)[o + tid] = 0x7fc00000u;
@@ -479,60 +524,111 @@ __global__ __launch_bounds__(256) void get_rows_kernel(const uint8_t *__restrict
         return;
     }
     const size_t nb = (size_t)id >> 7;
-    const int c = id & 127;
+    // the record's loads go out before the ids are counted
+    uint32_t w[K];
+    load_tile_row<K>(records, 1, k, n, kb * 8 + wave, nb * 8, lane, w);
+    const uint8_t *rec = records + (nb * (k >> 7) + kb) * group_bytes(K);
+    const uint16_t *su = (const uint16_t *)(rec + 2048 * K);
+    const uint16_t sua = su[lane], sub = su[lane + 64];
+    // the ids of the window in this column group, numbered in order
+    const bool match = w0 + tid < count && other >= 0 && (size_t)other < n && (size_t)(other >> 7) == nb;
+    const uint64_t ball = __builtin_amdgcn_ballot_w64(match);
+    const int below = __builtin_popcountll(ball & (((uint64_t)1 << lane) - 1));
+    if (lane == 0) matches[wave] = __builtin_popcountll(ball);
+    if (tid == self) member_row[0] = below;  // r's number within its wave, until the next barrier
+    __syncthreads();
+    int first = member_row[0], total = 0, before = 0;  // r's number, all matches, those of the waves before this one
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        const int m = __builtin_amdgcn_readfirstlane(matches[i]);
+        total += m;
+        if (i < (self >> 6)) first += m;
+        if (i < wave) before += m;
+    }
+    first = __builtin_amdgcn_readfirstlane(first);
+    if (first % kGetRowsShare) return;  // uniform: another workgroup serves r
+    const int nids = total - first < kGetRowsShare ? total - first : kGetRowsShare;
+    u4 frag[4];
+    decode_tile_row<K, CB>(w, lane, frag);
+    __syncthreads();  // member_row[0] has been read
+    const int at = before + below - first;
+    if (match && at >= 0 && at < kGetRowsShare) {
+        member_row[at] = tid;
+        member_col[at] = other & 127;
+    }
+    __syncthreads();
+    const int b = h128_lane_block(lane & 15);
+    uint32_t up1 = (b & 1) ? ~0u : 0u, up2 = (b & 2) ? ~0u : 0u, up4 = (b & 4) ? ~0u : 0u, up8 = (b & 8) ? ~0u : 0u;
+    asm("" : "+v"(up1), "+v"(up2), "+v"(up4), "+v"(up8));  // masks, not conditions
+    // this lane's row of the tile row: block bits 2, 1, 0 and the half of its row pair (bit 3)
+    const int row = 16 * wave + (up4 & 8) + (up2 & 4) + (up1 & 2) + (up8 & 1);
+    const float svc = half_bits_to_float(((const uint16_t *)(rec + 2048 * K + 256))[wave < nids ? member_col[wave] : 0]);
+    // the operands of stride 1, on packed row pairs: the same for every id
+    uint32_t own[4][2], got[4][2];
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+#pragma unroll
+        for (int vp = 0; vp < 2; ++vp) {
+            const uint32_t lo = vp ? frag[f].z : frag[f].x, hi = vp ? frag[f].w : frag[f].y;
+            own[f][vp] = pick(up1, lo, hi);
+            got[f][vp] = (uint32_t)__builtin_amdgcn_mov_dpp((int)pick(up1, hi, lo), 0xB1, 0xF, 0xF, false);
+        }
 #pragma unroll 1
-    for (int i = 0; i < 4; ++i) {
-        const int run = tid + 256 * i;
-        const int tile = run >> 4, rc = run & 15;
-        const int cr = rc & 7, h = rc >> 3, tr = tile >> 3, tc = tile & 7;
-        const uint32_t *tp = tile_ptr<K>(records, 1, k, n, kb * 8 + tr, nb * 8 + tc);
-        uint32_t w[RunGeo<K>::NW];
-        load_run_words<K>(tp, cr, h, w);
-        u4 a1, a2;
-        decode_run<K, CB>(w, a1, a2);
-        const uint32_t p1[4] = {a1.x, a1.y, a1.z, a1.w}, p2[4] = {a2.x, a2.y, a2.z, a2.w};
+    for (int q = 0; q < nids; ++q) {
+        const int c = __builtin_amdgcn_readfirstlane(member_col[q]);
+        float al[7];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r0 = tr * 16 + run_slot_row(h, 2 * v), r1 = tr * 16 + run_slot_row(h, 2 * v + 1);
-            const int cc = tc * 16 + cr;
-            blk[r0 * P + cc] = half_bits_to_float((uint16_t)(p1[v] & 0xffffu));
-            blk[r1 * P + cc] = half_bits_to_float((uint16_t)(p1[v] >> 16));
-            blk[r0 * P + cc + 8] = half_bits_to_float((uint16_t)(p2[v] & 0xffffu));
-            blk[r1 * P + cc + 8] = half_bits_to_float((uint16_t)(p2[v] >> 16));
+        for (int s = 0; s < 7; ++s) al[s] = (c >> s) & 1 ? -1.f : 1.f;
+#pragma unroll
+        for (int f = 0; f < 4; ++f)  // kept packed: hoisted out of the loop as 32 binary32 values they would spill
+            asm volatile("" : "+v"(own[f][0]), "+v"(own[f][1]), "+v"(got[f][0]), "+v"(got[f][1]));
+        float t[4][2][2];  // [f][row pair][row]: rows 8 (f % 2) + 4 pair + 2 b0 + row
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int vp = 0; vp < 2; ++vp)  // stride 1
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    t[f][vp][h] = __builtin_fmaf(half_bits_to_float((uint16_t)(own[f][vp] >> (16 * h))), al[0],
+                                                 half_bits_to_float((uint16_t)(got[f][vp] >> (16 * h))));
+        float e[4][2];  // stride 2: rows 8 (f % 2) + 4 b1 + 2 b0 + row
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) e[f][h] = fold_pair<2>(t[f][0][h], t[f][1][h], up2, al[1]);
+        float g[2][2];  // stride 4: rows 8 b2 + 4 b1 + 2 b0 + row, column half f / 2
+#pragma unroll
+        for (int ch = 0; ch < 2; ++ch)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) g[ch][h] = fold_pair<4>(e[2 * ch][h], e[2 * ch + 1][h], up4, al[2]);
+        float a[2];  // stride 8: the column halves
+#pragma unroll
+        for (int h = 0; h < 2; ++h) a[h] = __builtin_fmaf(g[1][h], al[3], g[0][h]);
+        float z = fold_pair<8>(a[0], a[1], up8, al[4]);  // stride 16: row pair split over b3
+        {  // strides 32, 64: every lane of the four 16-lane rows ends with the sum
+            const auto s32 = __builtin_amdgcn_permlane16_swap(__float_as_int(z), __float_as_int(z), false, false);
+            z = __builtin_fmaf(__int_as_float(s32[1]), al[5], __int_as_float(s32[0]));
+            const auto s64 = __builtin_amdgcn_permlane32_swap(__float_as_int(z), __float_as_int(z), false, false);
+            z = __builtin_fmaf(__int_as_float(s64[1]), al[6], __int_as_float(s64[0]));
         }
+        // the lower lane of a pair holds own +- hi negated where the stage subtracts
+        const uint32_t neg = ((c & 1) ? ~up1 : 0u) ^ ((c & 2) ? ~up2 : 0u) ^ ((c & 4) ? ~up4 : 0u) ^ ((c & 16) ? ~up8 : 0u);
+        const float scale = __uint_as_float(__float_as_uint(kScale) ^ (neg & 0x80000000u));
+        if (lane < 16) colv[q][row] = __builtin_fmaf(z, scale, 0.f);
     }
     __syncthreads();
-    // row tid: after the stage of stride 2^s only positions agreeing with c on
-    // bits 0..s matter; v[m] holds position (m << (s + 1)) | (c & (2^(s+1) - 1))
-    if (tid < 128) {
-        const float *row = blk + tid * P;
-        float v[64];
-#pragma unroll
-        for (int m = 0; m < 64; ++m) {
-            const float a = row[2 * m], b = row[2 * m + 1];
-            v[m] = (c & 1) ? a - b : a + b;
-        }
-#pragma unroll
-        for (int s = 1; s < 7; ++s)
-#pragma unroll
-            for (int m = 0; m < (64 >> s); ++m) v[m] = ((c >> s) & 1) ? v[2 * m] - v[2 * m + 1] : v[2 * m] + v[2 * m + 1];
-        colv[tid] = v[0] * 0.08838834764831844055f;
-    }
-    __syncthreads();
-    if (tid < 64) {
-        float e0 = colv[tid], e1 = colv[tid + 64];
-        h128_wave(e0, e1, tid);
-        const uint8_t *rec = records + (nb * (k >> 7) + kb) * group_bytes(K);
-        const uint16_t *su = (const uint16_t *)(rec + 2048 * K);
-        const float svc = half_bits_to_float(((const uint16_t *)(rec + 2048 * K + 256))[c]);
-        const uint16_t h0 = float_to_half_bits(mul_rn_f32(mul_rn_f32(e0, half_bits_to_float(su[tid])), svc));
-        const uint16_t h1 = float_to_half_bits(mul_rn_f32(mul_rn_f32(e1, half_bits_to_float(su[tid + 64])), svc));
+    if (wave < nids) {
+        float e0 = colv[wave][lane], e1 = colv[wave][lane + 64];
+        h128_wave(e0, e1, lane);
+        const uint16_t h0 = float_to_half_bits(mul_rn_f32(mul_rn_f32(e0, half_bits_to_float(sua)), svc));
+        const uint16_t h1 = float_to_half_bits(mul_rn_f32(mul_rn_f32(e1, half_bits_to_float(sub)), svc));
+        const size_t o = (w0 + member_row[wave]) * out_stride + kb * 128;
         if (out_f16) {
-            ((uint16_t *)out)[o + tid] = h0;
-            ((uint16_t *)out)[o + tid + 64] = h1;
+            ((uint16_t *)out)[o + lane] = h0;
+            ((uint16_t *)out)[o + lane + 64] = h1;
         } else {
-            ((float *)out)[o + tid] = half_bits_to_float(h0);
-            ((float *)out)[o + tid + 64] = half_bits_to_float(h1);
+            ((float *)out)[o + lane] = half_bits_to_float(h0);
+            ((float *)out)[o + lane + 64] = half_bits_to_float(h1);
         }
     }
 }
@@ -541,15 +637,16 @@ template <int K>
 static hipError_t launch_get_rows_k(const void *records, int cb, size_t k, size_t n, const int32_t *ids,
                                     size_t ids_stride, size_t count, void *out, int out_f16, size_t out_stride,
                                     int *bad_ids, hipStream_t stream) {
-    const dim3 grid((unsigned)count, (unsigned)(k / 128)), block(256);
+    const size_t gy = count < 32768 ? count : 32768;
+    const dim3 grid((unsigned)(k / 128), (unsigned)gy, (unsigned)((count + gy - 1) / gy)), block(kGetRowsThreads);
     const uint8_t *rec = (const uint8_t *)records;
     switch (cb) {
-    case 0: get_rows_kernel<K, 0><<<grid, block, 0, stream>>>(rec, k, n, ids, ids_stride, out, out_f16, out_stride,
-                                                                 bad_ids); break;
-    case 1: get_rows_kernel<K, 1><<<grid, block, 0, stream>>>(rec, k, n, ids, ids_stride, out, out_f16, out_stride,
-                                                                 bad_ids); break;
-    default: get_rows_kernel<K, 2><<<grid, block, 0, stream>>>(rec, k, n, ids, ids_stride, out, out_f16, out_stride,
-                                                                 bad_ids); break;
+    case 0: get_rows_kernel<K, 0><<<grid, block, 0, stream>>>(rec, k, n, ids, ids_stride, count, out, out_f16,
+                                                              out_stride, bad_ids); break;
+    case 1: get_rows_kernel<K, 1><<<grid, block, 0, stream>>>(rec, k, n, ids, ids_stride, count, out, out_f16,
+                                                              out_stride, bad_ids); break;
+    default: get_rows_kernel<K, 2><<<grid, block, 0, stream>>>(rec, k, n, ids, ids_stride, count, out, out_f16,
+                                                              out_stride, bad_ids); break;
     }
     return hipGetLastError();
 }
