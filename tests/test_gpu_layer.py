@@ -563,3 +563,63 @@ def test_every_tile_class_rate_and_codebook(amd, oracle, bits):
         for r, y, tag in ((rec, ys[0], "a"), (rec2, ys[1], "b")):
             ref = oracle.mul_mat(r, bits, cb, k, n, x, threads=THREADS)
             assert_layer_close(y.cpu().numpy(), ref, what=f"group {tag} bits={bits} cb={cb} rows=20")
+
+
+@pytest.mark.parametrize("rows,shapes", [(40, [512, 128, 384]), (100, [640, 1280]), (130, [256, 2048]),
+                                         (300, [1280, 128]), (530, [384, 512, 128, 640])])
+def test_group_gemm_one_launch_equals_single_calls(amd, oracle, rows, shapes):
+    """A grouped call above the GEMV rows: one GEMM launch whose matrices keep the splits each
+    has alone, so every output is mul_mat's bit for bit, with the workspace of documented size
+    and with one that only holds the calls one by one; strided outputs; fp16 and fp32."""
+    import torch
+    k, bits = 640, 3
+    recs = [dev(make_layer(1500 + i, k, n, bits)) for i, n in enumerate(shapes)]
+    print(f"  group gemm rows={rows} n={shapes}", flush=True)
+    for dt in (torch.float16, torch.float32):
+        x = torch.from_numpy(synth.activations(1510 + rows, rows, k)).cuda().to(dt)
+        single = [amd.mul_mat(r, bits, k, n, x, out_dtype=dt) for r, n in zip(recs, shapes)]
+        small = max([amd.workspace_bytes(k, n, rows) for n in shapes] + [amd.workspace_bytes(k, sum(shapes), rows)])
+        full = amd.group_workspace_bytes(k, shapes, rows)
+        assert full > small
+        for nbytes in (full, small):
+            ws = amd.new_workspace(k, shapes[0], rows, nbytes=nbytes)
+            ys = [torch.full((rows, n + 8 * i), 7.0, dtype=dt, device="cuda") for i, n in enumerate(shapes)]
+            amd.mul_mat_group([(r, n, y[:, :n]) for r, n, y in zip(recs, shapes, ys)], bits, k, x, workspace=ws)
+            for n, y, want in zip(shapes, ys, single):
+                assert torch.equal(y[:, :n], want) and bool((y[:, n:] == 7.0).all()), (dt, nbytes, n)
+    ref = oracle.mul_mat(make_layer(1500, k, shapes[0], bits), bits, 2, k, shapes[0],
+                         synth.activations(1510 + rows, rows, k))
+    assert_layer_close(single[0].cpu().numpy(), ref, what=f"group gemm rows={rows}")
+
+
+@pytest.mark.parametrize("rows,ns", [(260, [33024]), (260, [40960]), (600, [16640]), (260, [33024, 33152]),
+                                     (200, [33024]), (260, [33024, 128])])
+def test_gemm_tail_round_is_split(amd, oracle, rows, ns):
+    """More tiles than CUs: full rounds of whole tiles, the last round's tiles split over k
+    (258, 320 and 2 x 130 tiles), alone and in a group (258 + 259 tiles sharing one tail;
+    258 and 1 tile each with its own).  Columns on both sides of the cut against the oracle, every column against the
+    same columns computed as a narrower matrix (whose plan has no tail), and the call with a
+    workspace too small for the tail's partials."""
+    import torch
+    k, bits = 384, 4
+    layers = [make_layer(1600 + i, k, n, bits) for i, n in enumerate(ns)]
+    recs = [dev(r) for r in layers]
+    xh = synth.activations(1610 + rows, rows, k)
+    x = torch.from_numpy(xh).cuda()
+    print(f"  tail rows={rows} n={ns}", flush=True)
+    if len(ns) > 1:
+        ys = amd.mul_mat_group(list(zip(recs, ns)), bits, k, x)
+    else:
+        ys = [amd.mul_mat(recs[0], bits, k, ns[0], x)]
+    gb = synth.group_bytes(bits) * (k // 128)
+    for layer, rec, n, y in zip(layers, recs, ns, ys):
+        for g0 in range(0, n // 128, 64):
+            g1 = min(g0 + 64, n // 128)
+            part = rec.view(torch.uint8).reshape(-1)[g0 * gb: g1 * gb].contiguous()
+            want = amd.mul_mat(part, bits, k, 128 * (g1 - g0), x).cpu().numpy()
+            assert_layer_close(y[:, 128 * g0: 128 * g1].cpu().numpy(), want, what=f"columns {128 * g0}..")
+        raw = np.ascontiguousarray(layer).view(np.uint8).reshape(-1)
+        groups = sorted({0, n // 256, max(0, n // 128 - 4), n // 128 - 1})
+        for g in groups:
+            ref = oracle.mul_mat(raw[g * gb: (g + 1) * gb].copy(), bits, 2, k, 128, xh)
+            assert_layer_close(y[:, 128 * g: 128 * g + 128].cpu().numpy(), ref, what=f"group {g}")

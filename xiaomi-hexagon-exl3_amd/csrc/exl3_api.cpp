@@ -45,28 +45,101 @@ std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, InternalWs> g_ws;
 std::vector<void *> g_ws_retired;
 
-exl3_status internal_workspace(size_t need, hipStream_t stream, void **out) {
+// Calls f with the largest row count of each GEMM plan up to `rows` rows (a plan depends
+// on the tile height and the number of m-tiles; r_hi >= r, so every pass moves on).
+template <typename F>
+void for_gemm_plans(size_t rows, F f) {
+    for (size_t r = exl3k::kGemvSingleMaxRows + 1; r <= rows;) {
+        const int bm = exl3k::gemm_tile_rows(r);
+        size_t r_hi = std::min(rows, (r + bm - 1) / bm * bm);
+        while (exl3k::gemm_tile_rows(r_hi) != bm) --r_hi;
+        f(r_hi);
+        r = r_hi + 1;
+    }
+}
+
+// `want` bytes if the workspace may grow, else the `need` it must have; *bytes: what it has.
+exl3_status internal_workspace(size_t need, size_t want, hipStream_t stream, void **out, size_t *bytes) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return EXL3_HIP_ERROR;
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     InternalWs &ws = g_ws[std::make_pair(dev, stream)];
-    if (ws.bytes < need) {
+    if (ws.bytes < want) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(stream, &capture) != hipSuccess) return EXL3_HIP_ERROR;
-        if (capture != hipStreamCaptureStatusNone) return EXL3_WORKSPACE_TOO_SMALL;
-        const size_t bytes = std::max(need, 2 * ws.bytes);  // geometric growth bounds what is retired
-        void *p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) return EXL3_HIP_ERROR;
-        if (exl3k::launch_zero(p, bytes, stream) != hipSuccess) {
-            (void)hipFree(p);
-            return EXL3_HIP_ERROR;
+        if (capture != hipStreamCaptureStatusNone) {
+            if (ws.bytes < need) return EXL3_WORKSPACE_TOO_SMALL;
+        } else {
+            size_t grown = std::max(want, 2 * ws.bytes);  // geometric growth bounds what is retired
+            void *p = nullptr;
+            if (hipMalloc(&p, grown) != hipSuccess) {
+                p = nullptr;
+                (void)hipGetLastError();
+                if (ws.bytes < need) {  // the least will do
+                    grown = need;
+                    if (hipMalloc(&p, grown) != hipSuccess) return EXL3_HIP_ERROR;
+                }
+            }
+            if (p) {
+                if (exl3k::launch_zero(p, grown, stream) != hipSuccess) {
+                    (void)hipFree(p);
+                    return EXL3_HIP_ERROR;
+                }
+                if (ws.ptr) g_ws_retired.push_back(ws.ptr);
+                ws.ptr = p;
+                ws.bytes = grown;
+            }
         }
-        if (ws.ptr) g_ws_retired.push_back(ws.ptr);
-        ws.ptr = p;
-        ws.bytes = bytes;
     }
     *out = ws.ptr;
+    *bytes = ws.bytes;
     return EXL3_OK;
+}
+
+// A call's workspace: the caller's, of at least `need` bytes, or the internal one, of
+// want() bytes where it may grow.
+template <typename F>
+exl3_status call_workspace(size_t need, F want, hipStream_t stream, void **workspace, size_t *bytes) {
+    if (!*workspace) return internal_workspace(need, want(), stream, workspace, bytes);
+    if (!aligned(*workspace, 256)) return EXL3_INVAL_PARAMS;
+    return *bytes < need ? EXL3_WORKSPACE_TOO_SMALL : EXL3_OK;
+}
+
+// Largest plan over every row count 1..rows and both paths a row count can take
+// (rows 15..32: the GEMM for one matrix, the GEMV for a group of them), so that one
+// workspace serves all smaller calls of the same (k, n) in turn (every plan starts
+// with the same exchange region).
+size_t mul_mat_need(size_t k, size_t n, size_t rows, bool tails) {
+    if (!valid_matrix(k, n, 128) || rows < 1 || rows > kMaxRows) return 0;
+    size_t need = 0;
+    const size_t gemv_rows = rows < (size_t)exl3k::kGemvMaxRows ? rows : (size_t)exl3k::kGemvMaxRows;
+    for (size_t r = 1; r <= gemv_rows; ++r) {
+        const exl3k::GemvPlan p = exl3k::gemv_plan(k, n, r);
+        need = std::max(need, p.fits ? p.bytes : exl3k::gemm_plan(k, n, r, tails).bytes);
+    }
+    for_gemm_plans(rows, [&](size_t r) { need = std::max(need, exl3k::gemm_plan(k, n, r, tails).bytes); });
+    return need;
+}
+
+// The same for a grouped call: the least it takes (one GEMV launch over the total
+// width, or one call per matrix), and with `fused` the GEMM launch for all of them.
+size_t group_need(size_t k, const size_t *n, size_t count, size_t rows, bool fused) {
+    if (!n || count < 1 || count > (size_t)exl3k::kGemvMaxTargets) return 0;
+    size_t n_total = 0, need = 0;
+    for (size_t i = 0; i < count; ++i) {
+        const size_t b = mul_mat_need(k, n[i], rows, fused);
+        if (!b) return 0;
+        need = std::max(need, b);
+        n_total += n[i];
+    }
+    if (n_total > kMaxDim) return 0;
+    need = std::max(need, mul_mat_need(k, n_total, rows, fused));
+    if (fused && count > 1)
+        for_gemm_plans(rows, [&](size_t r) {
+            const exl3k::GemmPlan p = exl3k::gemm_plan_group(k, n, (int)count, r);
+            if (p.ok) need = std::max(need, p.bytes);
+        });
+    return need;
 }
 
 }  // namespace
@@ -182,29 +255,7 @@ int exl3_hip_supports_op(exl3_op op, const exl3_tensor_info *dst, const exl3_ten
     return 0;
 }
 
-// The largest plan over every row count 1..rows and both paths a row count can
-// take (rows 15..32: the GEMM for one matrix, the GEMV for a group of them), so
-// one workspace serves all smaller calls of the same (k, n) in turn (every plan
-// starts with the same exchange region).
-size_t exl3_hip_mul_mat_workspace_bytes(size_t k, size_t n, size_t rows) {
-    if (!valid_matrix(k, n, 128) || rows < 1 || rows > kMaxRows) return 0;
-    size_t need = 0;
-    const size_t gemv_rows = rows < (size_t)exl3k::kGemvMaxRows ? rows : (size_t)exl3k::kGemvMaxRows;
-    for (size_t r = 1; r <= gemv_rows; ++r) {
-        const exl3k::GemvPlan p = exl3k::gemv_plan(k, n, r);
-        need = std::max(need, p.fits ? p.bytes : exl3k::gemm_plan(k, n, r).bytes);
-    }
-    // GEMM plans: the largest row count of each (tile height, m-tile count) run;
-    // r_hi >= r, so every pass moves on
-    for (size_t r = exl3k::kGemvSingleMaxRows + 1; r <= rows;) {
-        const int bm = exl3k::gemm_tile_rows(r);
-        size_t r_hi = std::min(rows, (r + bm - 1) / bm * bm);
-        while (exl3k::gemm_tile_rows(r_hi) != bm) --r_hi;
-        need = std::max(need, exl3k::gemm_plan(k, n, r_hi).bytes);
-        r = r_hi + 1;
-    }
-    return need;
-}
+size_t exl3_hip_mul_mat_workspace_bytes(size_t k, size_t n, size_t rows) { return mul_mat_need(k, n, rows, true); }
 
 exl3_status exl3_hip_workspace_init(void *workspace, size_t workspace_bytes, hipStream_t stream) {
     if (!workspace) {  // the internal workspace of (current device, stream), if there is one
@@ -255,23 +306,25 @@ static exl3_status mul_mat_impl(const void *records, unsigned bits, unsigned cod
     if (!records || !x || !y || !aligned(records, 16)) return EXL3_INVAL_PARAMS;
     if (!aligned(x, dtype_size(xt)) || !aligned(y, dtype_size(yt))) return EXL3_INVAL_PARAMS;
     if (x_row_stride < k || y_row_stride < n) return EXL3_INVAL_PARAMS;
-    const bool gemv = exl3k::gemv_serves_single(k, n, rows);
-    const size_t need = exl3_hip_mul_mat_workspace_bytes(k, n, rows);
-    if (workspace) {
-        if (!aligned(workspace, 256)) return EXL3_INVAL_PARAMS;
-        if (workspace_bytes < need) return EXL3_WORKSPACE_TOO_SMALL;
-    } else {
-        const exl3_status st = internal_workspace(need, stream, &workspace);
-        if (st != EXL3_OK) return st;
-    }
+    const exl3_status st = call_workspace(mul_mat_need(k, n, rows, false), [&] { return mul_mat_need(k, n, rows, true); },
+                                          stream, &workspace, &workspace_bytes);
+    if (st != EXL3_OK) return st;
+    exl3k::GemvTargets tg{};
+    tg.records[0] = (const uint8_t *)records;
+    tg.y[0] = y;
+    tg.y_stride[0] = y_row_stride;
+    tg.res[0] = res;
+    tg.res_stride[0] = res_row_stride;
+    tg.nb_end[0] = (int)(n / 128);
+    tg.count = 1;
     const int xf = xt == EXL3_F16, yf = yt == EXL3_F16;
-    if (gemv)
-        return from_hip(exl3k::launch_gemv(records, (int)bits, (int)codebook, k, n, x, xf, rows, x_row_stride, y, yf,
-                                           y_row_stride, workspace, exl3k::gemv_plan(k, n, rows), stream, res,
-                                           res_row_stride));
-    return from_hip(exl3k::launch_gemm(records, (int)bits, (int)codebook, k, n, x, xf, rows, x_row_stride, y, yf,
-                                       y_row_stride, workspace, exl3k::gemm_plan(k, n, rows), stream, res,
-                                       res_row_stride));
+    if (exl3k::gemv_serves_single(k, n, rows))
+        return from_hip(exl3k::launch_gemv_targets(tg, (int)bits, (int)codebook, x, xf, rows, x_row_stride, yf,
+                                                   workspace, exl3k::gemv_plan(k, n, rows), stream));
+    exl3k::GemmPlan plan = exl3k::gemm_plan(k, n, rows, true);
+    if (plan.bytes > workspace_bytes) plan = exl3k::gemm_plan(k, n, rows, false);
+    return from_hip(exl3k::launch_gemm_targets(tg, (int)bits, (int)codebook, x, xf, rows, x_row_stride, yf, workspace,
+                                               plan, stream));
 }
 
 exl3_status exl3_hip_mul_mat(const void *records, unsigned bits, unsigned codebook, size_t k, size_t n, const void *x,
@@ -316,26 +369,13 @@ exl3_status exl3_hip_mul_mat_group(const exl3_matrix_desc *mats, size_t count, u
     // enqueued, for whichever of the two paths below the call takes
     size_t ns[exl3k::kGemvMaxTargets];
     for (size_t i = 0; i < count; ++i) ns[i] = mats[i].n;
-    const size_t need = exl3_hip_mul_mat_group_workspace_bytes(k, ns, count, rows);
-    if (workspace) {
-        if (!aligned(workspace, 256)) return EXL3_INVAL_PARAMS;
-        if (workspace_bytes < need) return EXL3_WORKSPACE_TOO_SMALL;
-    } else {
-        const exl3_status st = internal_workspace(need, stream, &workspace);
-        if (st != EXL3_OK) return st;
-        workspace_bytes = need;
-    }
-    // GEMM (or, for one matrix above the single-matrix GEMV rows, whichever
-    // exl3_hip_mul_mat picks): one call per matrix, each a full-size launch
-    if (!exl3k::gemv_serves(k, n_total, rows) || (count == 1 && !exl3k::gemv_serves_single(k, n_total, rows))) {
-        for (size_t i = 0; i < count; ++i) {
-            const exl3_status st = exl3_hip_mul_mat(mats[i].records, bits, codebook, k, mats[i].n, x, xt, rows,
-                                                    x_row_stride, mats[i].y, yt, mats[i].y_row_stride, workspace,
-                                                    workspace_bytes, stream);
-            if (st != EXL3_OK) return st;
-        }
-        return EXL3_OK;
-    }
+    const exl3_status st = call_workspace(group_need(k, ns, count, rows, false),
+                                          [&] { return group_need(k, ns, count, rows, true); }, stream, &workspace,
+                                          &workspace_bytes);
+    if (st != EXL3_OK) return st;
+    if (count == 1)
+        return exl3_hip_mul_mat(mats[0].records, bits, codebook, k, mats[0].n, x, xt, rows, x_row_stride, mats[0].y,
+                                yt, mats[0].y_row_stride, workspace, workspace_bytes, stream);
     exl3k::GemvTargets tg{};
     int nb_end = 0;
     for (size_t i = 0; i < count; ++i) {
@@ -346,21 +386,29 @@ exl3_status exl3_hip_mul_mat_group(const exl3_matrix_desc *mats, size_t count, u
         tg.nb_end[i] = nb_end;
     }
     tg.count = (int)count;
-    return from_hip(exl3k::launch_gemv_targets(tg, (int)bits, (int)codebook, x, xt == EXL3_F16, rows, x_row_stride,
-                                               yt == EXL3_F16, workspace, exl3k::gemv_plan(k, n_total, rows), stream));
+    const int xf = xt == EXL3_F16, yf = yt == EXL3_F16;
+    if (exl3k::gemv_serves(k, n_total, rows))
+        return from_hip(exl3k::launch_gemv_targets(tg, (int)bits, (int)codebook, x, xf, rows, x_row_stride, yf,
+                                                   workspace, exl3k::gemv_plan(k, n_total, rows), stream));
+    bool gemm = true;  // every matrix alone would run the GEMM
+    for (size_t i = 0; i < count; ++i) gemm = gemm && !exl3k::gemv_serves_single(k, ns[i], rows);
+    if (gemm) {
+        const exl3k::GemmPlan plan = exl3k::gemm_plan_group(k, ns, (int)count, rows);
+        if (plan.ok && plan.bytes <= workspace_bytes)
+            return from_hip(exl3k::launch_gemm_targets(tg, (int)bits, (int)codebook, x, xf, rows, x_row_stride, yf,
+                                                       workspace, plan, stream));
+    }
+    for (size_t i = 0; i < count; ++i) {  // mixed kernels or a smaller workspace: one call per matrix
+        const exl3_status each = exl3_hip_mul_mat(mats[i].records, bits, codebook, k, mats[i].n, x, xt, rows,
+                                                  x_row_stride, mats[i].y, yt, mats[i].y_row_stride, workspace,
+                                                  workspace_bytes, stream);
+        if (each != EXL3_OK) return each;
+    }
+    return EXL3_OK;
 }
 
 size_t exl3_hip_mul_mat_group_workspace_bytes(size_t k, const size_t *n, size_t count, size_t rows) {
-    if (!n || count < 1 || count > (size_t)exl3k::kGemvMaxTargets) return 0;
-    size_t n_total = 0, need = 0;
-    for (size_t i = 0; i < count; ++i) {
-        const size_t b = exl3_hip_mul_mat_workspace_bytes(k, n[i], rows);
-        if (!b) return 0;
-        need = std::max(need, b);  // the per-matrix calls of the GEMM path
-        n_total += n[i];
-    }
-    if (n_total > kMaxDim) return 0;
-    return std::max(need, exl3_hip_mul_mat_workspace_bytes(k, n_total, rows));  // the one GEMV launch
+    return group_need(k, n, count, rows, true);
 }
 
 exl3_status exl3_hip_mul_mat_nd(const void *records, unsigned bits, unsigned codebook, size_t k, size_t n,
@@ -378,15 +426,11 @@ exl3_status exl3_hip_mul_mat_nd(const void *records, unsigned bits, unsigned cod
     const size_t rows = view_rows(x_info);
     if (!exl3_hip_supports_mul_mat(bits, codebook, k, n, rows, xt, yt) || !records || !x || !y)
         return EXL3_INVAL_PARAMS;
-    const size_t need = exl3_hip_mul_mat_workspace_bytes(k, n, rows);  // every call below needs at most this
-    if (workspace) {
-        if (!aligned(workspace, 256)) return EXL3_INVAL_PARAMS;
-        if (workspace_bytes < need) return EXL3_WORKSPACE_TOO_SMALL;
-    } else {
-        const exl3_status st = internal_workspace(need, stream, &workspace);
-        if (st != EXL3_OK) return st;
-        workspace_bytes = need;
-    }
+    // every call below needs at most this
+    const exl3_status wst = call_workspace(mul_mat_need(k, n, rows, false),
+                                           [&] { return mul_mat_need(k, n, rows, true); }, stream, &workspace,
+                                           &workspace_bytes);
+    if (wst != EXL3_OK) return wst;
     // Row dimensions 1, 2, 3 in order join one run while both views step through
     // them with one row stride (a run's stride at least a row, as exl3_hip_mul_mat
     // takes it); the run is one call, the dimensions from `outer` on loop.
@@ -559,13 +603,13 @@ exl3_status exl3_hip_pack_records(const uint16_t *packed, const uint16_t *su, co
 
 // Workspace of exl3_hip_iface_matmul: the mul_mat workspace (its counters first,
 // so one zero-fill covers both), then the packed records.
-static size_t iface_records_offset(size_t k, size_t n, size_t batch) {
-    return (exl3_hip_mul_mat_workspace_bytes(k, n, batch) + 255) & ~(size_t)255;
+static size_t iface_records_offset(size_t k, size_t n, size_t batch, bool tails) {
+    return (mul_mat_need(k, n, batch, tails) + 255) & ~(size_t)255;
 }
 
 size_t exl3_hip_iface_matmul_workspace_bytes(unsigned bits, size_t k, size_t n, size_t batch) {
     if (bits < 1 || bits > 8 || !valid_matrix(k, n, 128) || batch < 1 || batch > kMaxRows) return 0;
-    return iface_records_offset(k, n, batch) + (n / 128) * (k / 128) * ((size_t)2048 * bits + 512);
+    return iface_records_offset(k, n, batch, true) + (n / 128) * (k / 128) * ((size_t)2048 * bits + 512);
 }
 
 // exl3_iface_matmul (src/hexagon/exl3_service.c:265-305): the argument checks of
@@ -578,17 +622,14 @@ exl3_status exl3_hip_iface_matmul(unsigned bits, unsigned codebook, size_t k, si
     if (!packed || !suh || !svh || !x || !y) return EXL3_INVAL_PARAMS;
     if (!aligned(packed, 16) || !aligned(suh, 16) || !aligned(svh, 16) || !aligned(x, 4) || !aligned(y, 4))
         return EXL3_INVAL_PARAMS;
-    const size_t need = exl3_hip_iface_matmul_workspace_bytes(bits, k, n, batch);
-    if (workspace) {
-        if (!aligned(workspace, 256)) return EXL3_INVAL_PARAMS;
-        if (workspace_bytes < need) return EXL3_WORKSPACE_TOO_SMALL;
-    } else {
-        const exl3_status st = internal_workspace(need, stream, &workspace);
-        if (st != EXL3_OK) return st;
-    }
-    const size_t roff = iface_records_offset(k, n, batch);
+    const size_t want = exl3_hip_iface_matmul_workspace_bytes(bits, k, n, batch);
+    const size_t least = iface_records_offset(k, n, batch, false);
+    const size_t need = least + (want - iface_records_offset(k, n, batch, true));
+    exl3_status st = call_workspace(need, [&] { return want; }, stream, &workspace, &workspace_bytes);
+    if (st != EXL3_OK) return st;
+    const size_t roff = workspace_bytes < want ? least : iface_records_offset(k, n, batch, true);
     void *records = (uint8_t *)workspace + roff;
-    exl3_status st = exl3_hip_pack_records(packed, suh, svh, bits, k, n, records, stream);
+    st = exl3_hip_pack_records(packed, suh, svh, bits, k, n, records, stream);
     if (st != EXL3_OK) return st;
     return exl3_hip_mul_mat(records, bits, codebook, k, n, x, EXL3_F32, batch, k, y, EXL3_F32, n, workspace, roff,
                             stream);
@@ -603,3 +644,5 @@ exl3_status exl3_hip_validate_records(const void *records, size_t nbytes, unsign
 }
 
 }  // extern "C"
+
+size_t exl3k::mul_mat_least_workspace(size_t k, size_t n, size_t rows) { return mul_mat_need(k, n, rows, false); }

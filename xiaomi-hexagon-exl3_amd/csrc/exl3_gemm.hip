@@ -27,7 +27,7 @@ __host__ __device__ inline size_t gemm_xh_offset(int row, int kb, int e, int kbs
     const int ln = (row & 31) + 32 * (kk >> 3);
     return ((((size_t)(row >> 5) * kbs + kb) * 8 + ks) * 64 + ln) * 8 + (kk & 7);
 }
-// Workgroup (kb, 4 rb + wave) is one wave of 8 rows (two passes of 4; one wave
+// Workgroup (kb, 4 rb + wave, target) is one wave of 8 rows (two passes of 4; one wave
 // per workgroup spreads a short prep over more CUs than 4-wave workgroups:
 // -0.1 to -0.35 us per call at 24..512 rows); lane 16 g + l holds elements
 // 8 i .. 8 i + 7, i = h128_lane_block(l), of row 32 rb + 8 wave + 4 pass + g.  H128 stages 1, 2 and 4 are inside the lane, 8 .. 64 pair it with the
@@ -48,9 +48,18 @@ __device__ __forceinline__ void xprep_load(const void *__restrict__ x, const siz
         }
     }
 }
-__global__ __launch_bounds__(64) void gemm_xprep_kernel(const uint8_t *__restrict__ records, int bits,
-                                                         const void *__restrict__ x, int x_f16, size_t x_stride,
-                                                         int rows, int kbs, uint16_t *__restrict__ xh16) {
+// blockIdx.z: the target (its own su and its own copy of the activations, xh_stride
+// halves apart); ONE: a single target.
+template <bool ONE>
+__global__ __launch_bounds__(64) void gemm_xprep_kernel(GemvTargets tg, int bits, const void *__restrict__ x,
+                                                         int x_f16, size_t x_stride, int rows, int kbs,
+                                                         uint16_t *__restrict__ xh16, size_t xh_stride) {
+    const uint8_t *records = tg.records[0];
+    if constexpr (!ONE) {
+#pragma unroll
+        for (int i = 1; i < kGemvMaxTargets; ++i) records = (int)blockIdx.z == i ? tg.records[i] : records;
+        xh16 += blockIdx.z * xh_stride;
+    }
     // i: this lane's 8-element block of the row (h128_lane_block order)
     const int lane = threadIdx.x & 63, wave = blockIdx.y & 3, g = lane >> 4, i = h128_lane_block(lane & 15);
     const int kb = blockIdx.x, rb = blockIdx.y >> 2;
@@ -138,6 +147,56 @@ __global__ __launch_bounds__(64) void gemm_xprep_kernel(const uint8_t *__restric
 // (src/exl3-ggml.cpp:84-90); with one, gemm_reduce_kernel sums the partials in
 // split order and does the same.
 constexpr int kGemmTargetWgs = 256;  // one workgroup per CU (the accumulators fill the register file)
+
+// What column group nb (over all targets of the call) belongs to.
+struct GemmColumn {
+    const uint8_t *colgroup;  // its records
+    void *y;
+    const void *res;
+    size_t y_stride, res_stride;
+    int target, nb;  // nb within the target
+};
+// (Static indexes and selects here and below: the kernel arguments then arrive in a few
+// wide scalar loads, all at once; loads at computed indexes, one behind the other, cost
+// 1.3 us per call at M = 512.)
+template <bool ONE>
+__device__ __forceinline__ GemmColumn gemm_column(const GemvTargets &tg, int nb, size_t colgroup_bytes) {
+    GemmColumn c{tg.records[0], tg.y[0], tg.res[0], tg.y_stride[0], tg.res_stride[0], 0, nb};
+#pragma unroll
+    for (int i = 1; i < (ONE ? 1 : kGemvMaxTargets); ++i) {
+        const bool in = i < tg.count && nb >= tg.nb_end[i - 1];
+        c.colgroup = in ? tg.records[i] : c.colgroup;
+        c.y = in ? tg.y[i] : c.y;
+        c.res = in ? tg.res[i] : c.res;
+        c.y_stride = in ? tg.y_stride[i] : c.y_stride;
+        c.res_stride = in ? tg.res_stride[i] : c.res_stride;
+        c.target = in ? i : c.target;
+        c.nb = in ? nb - tg.nb_end[i - 1] : c.nb;
+    }
+    c.colgroup += (size_t)c.nb * colgroup_bytes;
+    return c;
+}
+// The segment whose `begin` (workgroups of the GEMM) or `unit0` (of the reduction) is the
+// last one at or below id.
+template <bool UNIT>
+__device__ __forceinline__ GemmSegment gemm_segment(const GemmGrid &gg, int id) {
+    GemmSegment s = gg.seg[0];
+#pragma unroll
+    for (int i = 1; i < kGemmMaxSegments; ++i) {
+        const GemmSegment &c = gg.seg[i];
+        const bool in = i < gg.count && id >= (UNIT ? c.unit0 : c.begin);
+        s.begin = in ? c.begin : s.begin;
+        s.nb0 = in ? c.nb0 : s.nb0;
+        s.tile0 = in ? c.tile0 : s.tile0;
+        s.tiles = in ? c.tiles : s.tiles;
+        s.splits = in ? c.splits : s.splits;
+        s.kq = in ? c.kq : s.kq;
+        s.kr = in ? c.kr : s.kr;
+        s.part0 = in ? c.part0 : s.part0;
+        s.unit0 = in ? c.unit0 : s.unit0;
+    }
+    return s;
+}
 
 __device__ __forceinline__ int gemm_w_offset(int n, int chunk) {  // halves
     return n * 128 + ((chunk ^ (n & 15)) << 3);
@@ -235,9 +294,8 @@ __device__ __forceinline__ void gemm_rows_out(float (&t)[4][NE], int lane, int r
 // split (its epilogue writes partials only).
 template <int K, int CB, int RB, int W, int NSG, int XD, int CH>
 __global__ __launch_bounds__(W * 64) void gemm_kernel(
-    const uint8_t *__restrict__ records, int kbs, int nbs, int mtiles, int splits, int kq, int kr,
-    const uint16_t *__restrict__ xh16, size_t k, uint16_t *__restrict__ partials, int *__restrict__ exps, void *y,
-    int y_f16, size_t y_stride, int rows, const void *res, size_t res_stride) {
+    GemvTargets tg, GemmGrid gg, const uint16_t *__restrict__ xh16, size_t xh_stride, uint16_t *__restrict__ partials,
+    int *__restrict__ exps, int y_f16, int rows) {
     constexpr int WR = W / CH;   // waves along the rows
     constexpr int NCB = 4 / CH;  // 32-column accumulator blocks per row block of a wave
     constexpr int BM = 32 * RB * WR;
@@ -250,20 +308,24 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
     const int rw = wave % WR, ch = wave / WR;  // row wave, column half
     const int lg = lane >> 4, li = lane & 15, j = li & 7;
     const int l32 = lane & 31, lh = lane >> 5;
+    // The segment of the grid this workgroup belongs to, and its item there.
     // Workgroups are dispatched to the 8 XCDs round-robin (blockIdx % 8) and each
-    // XCD has its own L2: renumber so that XCD x runs the contiguous range
-    // [x G / 8, (x + 1) G / 8) of the order (split, column group, m-tile), m-tile
-    // fastest.  The m-tiles of one column group then share its weight records,
-    // and the column groups of one split share its activation rows, in one L2.
-    const int G = gridDim.x;
-    int L = (G & 7) ? (int)blockIdx.x : (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3);
-    const int s = L / (mtiles * nbs);
-    L -= s * mtiles * nbs;
-    const int nb = L / mtiles, mt = L - nb * mtiles;
-    const int tile = mt * nbs + nb;
+    // XCD has its own L2: renumber so that XCD x runs a contiguous eighth of the
+    // segment's order (split, tile).  The m-tiles of one column group then share its
+    // weight records, and the column groups of one split share its activation rows,
+    // in one L2.  (A segment's begin is a multiple of 8, its ids are padded to one.)
+    const GemmSegment sg = gemm_segment<false>(gg, (int)blockIdx.x);
+    const int id = (int)blockIdx.x - sg.begin, items = sg.tiles * sg.splits, per_xcd = (items + 7) >> 3;
+    const int item = (id & 7) * per_xcd + (id >> 3);
+    if (item >= items) return;  // padding, whole workgroups
+    const int splits = sg.splits, s = splits > 1 ? item / sg.tiles : 0, ts = item - s * sg.tiles;
+    const int nbt = (sg.tile0 + ts) / gg.mtiles, mt = sg.tile0 + ts - nbt * gg.mtiles;
+    const int kbs = gg.kbs;
+    const GemmColumn col = gemm_column<false>(tg, sg.nb0 + nbt, (size_t)kbs * GB);
     // split s owns kq + (s < kr) records from kb0 (kq = kbs / splits, kr = kbs % splits, from the host)
-    const int kb0 = s * kq + (s < kr ? s : kr), kb1 = kb0 + kq + (s < kr ? 1 : 0);
-    const uint8_t *colgroup = records + (size_t)nb * kbs * GB;
+    const int kb0 = s * sg.kq + (s < sg.kr ? s : sg.kr), kb1 = kb0 + sg.kq + (s < sg.kr ? 1 : 0);
+    const uint8_t *colgroup = col.colgroup;
+    const size_t pblk = (size_t)sg.part0 + (size_t)ts * splits + s;  // this item's partial block
 
     // weights: this wave decodes groups q = H wave + h (h < H) of every record
     uint32_t wlane[H];
@@ -300,7 +362,7 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
     };
     // activations: A fragment (ks, rb) = the contiguous kilobyte of row block
     // (BM mt + 32 (RB rw + rb)) / 32, record kb, k-step ks (gemm_xh_offset)
-    const uint16_t *xblk = xh16 + ((size_t)(mt * BM / 32 + RB * rw) * kbs * 8 * 64 + lane) * 8;
+    const uint16_t *xblk = xh16 + col.target * xh_stride + ((size_t)(mt * BM / 32 + RB * rw) * kbs * 8 * 64 + lane) * 8;
     auto load_x_step = [&](int kb, int ks, h8 (&xs)[RB]) {
         const uint16_t *p = xblk + ((size_t)(kb < kb1 ? kb : kb1 - 1) * 8 + ks) * 512;
 #pragma unroll
@@ -414,7 +476,7 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
     // epilogue.  acc[rb][cb][e]: row 32 RB rw + 32 rb + (e % 4) + 8 (e / 4) + 4 lh,
     // column 32 (NCB ch + cb) + l32
     if (splits > 1) {
-        // fp16 partials in accumulator layout [tile][split][rw][rb][column block][vp]
+        // fp16 partials in accumulator layout [segment][tile][split][rw][rb][column block][vp]
         // [lane] x 16 bytes: elements 8 vp .. 8 vp + 7 of a 32x32 block (rows of
         // v = 2 vp, 2 vp + 1), summed in fp32 by gemm_reduce_kernel.  Each 32x32
         // block is stored scaled by 2^-e, e = exps[(tile, split, rw, rb, block)]
@@ -423,7 +485,7 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
         // fp16 keeps the layer within its tolerance (rel-L2 2.9e-4 against 2.1e-4
         // for fp32 partials with fp16 output, at k = 14336) for half the bytes.
         constexpr size_t kPerSplit = (size_t)WR * RB * 4 * 2 * 64 * 8;  // halves
-        uint16_t *dst = partials + ((size_t)tile * splits + s) * kPerSplit + (size_t)rw * RB * 8 * 512 + lane * 8;
+        uint16_t *dst = partials + pblk * kPerSplit + (size_t)rw * RB * 8 * 512 + lane * 8;
         auto pk = [](float a, float b, int e) {
             return (uint32_t)float_to_half_bits(__builtin_amdgcn_ldexpf(a, -e)) |
                    ((uint32_t)float_to_half_bits(__builtin_amdgcn_ldexpf(b, -e)) << 16);
@@ -438,7 +500,7 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
                 for (int e = 0; e < 16; ++e) m = fmaxf(m, fabsf(acc[rb][cb][e]));
                 m = wave_max(m);
                 const int ex = __builtin_amdgcn_frexp_expf(m) - 14;  // m < 2^(ex + 14); 0 (and Inf, NaN): -14
-                if (lane == 0) exps[(((size_t)tile * splits + s) * (WR * RB) + rw * RB + rb) * 4 + cg] = ex;
+                if (lane == 0) exps[(pblk * (WR * RB) + rw * RB + rb) * 4 + cg] = ex;
 #pragma unroll
                 for (int vp = 0; vp < 2; ++vp) {
                     const f16v &a = acc[rb][cb];
@@ -458,8 +520,8 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
             for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) t[cb][e] = acc[rb][cb][e];
-            gemm_rows_out<16>(t, lane, mt * BM + 32 * RB * rw + 32 * rb, svp, rows, y, y_f16, y_stride,
-                              (size_t)nb * 128, res, res_stride);
+            gemm_rows_out<16>(t, lane, mt * BM + 32 * RB * rw + 32 * rb, svp, rows, col.y, y_f16, col.y_stride,
+                              (size_t)col.nb * 128, col.res, col.res_stride);
         }
     }
 }
@@ -472,22 +534,27 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
 // of a batch in flight together; the sums go through LDS as [row][column], and wave w then
 // finishes rows 4 w .. 4 w + 3 (h128_wave over the 128 columns, sv, the optional
 // residual), lane l writing columns l and l + 64.
-template <int RB, int W, int SB>
-__global__ __launch_bounds__(256) void gemm_reduce_kernel(const uint16_t *__restrict__ partials,
-                                                          const int *__restrict__ exps, int splits, int nbs,
-                                                          const uint8_t *__restrict__ records, int bits, int kbs,
-                                                          void *y, int y_f16, size_t y_stride, int rows, int nunits,
-                                                          const void *res, size_t res_stride) {
+// ONE: a single target and a single split segment, gg.seg[0] (the other arguments stay
+// unread: with the general form -0.2 to -0.5 us per call at M = 512 and rows 37).
+template <int RB, int W, int SB, bool ONE>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemvTargets tg, GemmGrid gg, int bits,
+                                                          const uint16_t *__restrict__ partials,
+                                                          const int *__restrict__ exps, int y_f16, int rows) {
     constexpr int BM = 32 * RB * W;
     constexpr size_t kPerSplit = (size_t)W * RB * 4 * 2 * 64 * 8;  // halves
     __shared__ float sums[16][129];  // [row][column], padded against bank conflicts
     const int lane = threadIdx.x & 63, c = threadIdx.x >> 6;
-    const int u = blockIdx.x;
-    if (u >= nunits) return;  // whole workgroups
-    const int vp = u & 1, blk = (u >> 1) % (W * RB), tile = (u >> 1) / (W * RB);
-    const int mt = tile / nbs, nb = tile - mt * nbs;
-    const uint16_t *src = partials + (size_t)tile * splits * kPerSplit + (size_t)blk * 8 * 512 + (c * 2 + vp) * 512 +
-                          lane * 8;
+    const GemmSegment sg = ONE ? gg.seg[0] : gemm_segment<true>(gg, (int)blockIdx.x);
+    const int splits = sg.splits, u = (int)blockIdx.x - sg.unit0;
+    const int vp = u & 1, blk = (u >> 1) % (W * RB), ts = (u >> 1) / (W * RB);
+    const int nbt = (sg.tile0 + ts) / gg.mtiles, mt = sg.tile0 + ts - nbt * gg.mtiles;
+    const GemmColumn col = gemm_column<ONE>(tg, sg.nb0 + nbt, (size_t)gg.kbs * group_bytes(bits));
+    const int nb = col.nb;
+    void *y = col.y;
+    const void *res = col.res;
+    const size_t y_stride = col.y_stride, res_stride = col.res_stride;
+    const size_t pblk = (size_t)sg.part0 + (size_t)ts * splits;
+    const uint16_t *src = partials + pblk * kPerSplit + (size_t)blk * 8 * 512 + (c * 2 + vp) * 512 + lane * 8;
     float t[8];
 #pragma unroll 1
     for (int sp0 = 0; sp0 < splits; sp0 += SB) {
@@ -496,7 +563,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const uint16_t *__rest
 #pragma unroll
         for (int q = 0; q < SB; ++q) {
             const int sp = sp0 + q < splits ? sp0 + q : splits - 1;
-            ex[q] = exps[(((size_t)tile * splits + sp) * (W * RB) + blk) * 4 + c];
+            ex[q] = exps[((pblk + sp) * (W * RB) + blk) * 4 + c];
             // non-temporal loads for the partials of tiles up to 256 rows (each is
             // read once: k = 14336, n = 4096 rows 100..200 -0.7 to -1.6 us per call,
             // rows 16..64 -0.1 to -0.4 us, k = 2048, n = 6144 rows 256 -3.1 us); the
@@ -525,7 +592,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const uint16_t *__rest
 #pragma unroll
     for (int e = 0; e < 8; ++e) sums[(e & 3) + 8 * (e >> 2) + 4 * (lane >> 5)][32 * c + (lane & 31)] = t[e];
     __syncthreads();
-    const uint16_t *svp = (const uint16_t *)(records + (size_t)nb * kbs * group_bytes(bits) + 2048 * bits + 256);
+    const uint16_t *svp = (const uint16_t *)(col.colgroup + 2048 * bits + 256);
     const float sv0 = half_bits_to_float(svp[lane]), sv1 = half_bits_to_float(svp[lane + 64]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -572,8 +639,8 @@ int gemm_tile_rows(size_t rows) {
     return rows <= 32 ? 32 : rows <= 64 ? 64 : rows <= 128 ? 128 : rows <= 256 ? 256 : 512;
 }
 
-// k splits of a tile class: split k only below kGemmSplitTiles tiles (the split
-// partials are summed by gemm_reduce_kernel), at most one split per record.
+// k splits of a set of `tiles` tiles that run together (summed by gemm_reduce_kernel),
+// at most one split per record.
 // 32- and 64-row tiles fill the CUs once (one workgroup each); 32-row tiles (4
 // waves, 64 KB of LDS) run two per CU when each split keeps >= 4 records (rows
 // 17..32 at k = 14336, n = 4096: 22.7 -> 21.2 us; at k <= 6144 two per CU with
@@ -586,9 +653,9 @@ int gemm_tile_rows(size_t rows) {
 // least 4 records per split it takes k = 2048, n = 512 at rows 300 from 23.4
 // to 18.8 us and k = 2048, n = 2048 at rows 24 from 13.7 to 11.6 us.
 static int gemm_splits(int kbs, int tiles, int bm) {
-    if (tiles >= (int)kGemmSplitTiles) return 1;
     int s;
     if (bm <= 64) {
+        if (tiles >= (int)kGemmSplitTiles) return 1;
         int wgs = kGemmTargetWgs;
         if (bm == 32 && kbs / ((2 * kGemmTargetWgs + tiles - 1) / tiles) >= 4) wgs = 2 * kGemmTargetWgs;
         s = 2 * tiles > wgs ? (wgs + tiles - 1) / tiles : wgs / tiles;
@@ -610,115 +677,178 @@ static int gemm_splits(int kbs, int tiles, int bm) {
     return s < 1 ? 1 : (s > kbs ? kbs : s);
 }
 
-static GemmPlan gemm_plan_bm(size_t k, size_t n, size_t rows, int bm) {
+// Appends the segments of `tiles` tiles over column groups nb0 .. nb0 + nbs - 1: one
+// without a split, or one with, or (tails, 256- and 512-row tiles, more tiles than CUs)
+// the full rounds of one tile per CU without and the last, partial round's tiles with a
+// split that fills the CUs again, where gemm_splits finds one cheaper than a whole round.
+static void gemm_add(GemmPlan &p, GemmSegment *direct, int &nd, GemmSegment *split, int &ns, int nb0, int nbs,
+                     bool tails) {
+    const int tiles = nbs * p.mtiles;
+    int full = 0, s = gemm_splits(p.kbs, tiles, p.bm);
+    if (s == 1) full = tiles;
+    if (tails && p.bm >= 256 && tiles > kGemmTargetWgs && tiles % kGemmTargetWgs) {
+        const int t = gemm_splits(p.kbs, tiles % kGemmTargetWgs, p.bm);
+        if (t > 1) s = t, full = tiles - tiles % kGemmTargetWgs;
+    }
+    GemmSegment g{};
+    g.nb0 = nb0;
+    if (full) {
+        g.tile0 = 0;
+        g.tiles = full;
+        g.splits = 1;
+        g.kq = p.kbs;
+        direct[nd++] = g;
+    }
+    if (full < tiles) {
+        g.tile0 = full;
+        g.tiles = tiles - full;
+        g.splits = s;
+        g.kq = p.kbs / s;
+        g.kr = p.kbs % s;
+        split[ns++] = g;
+    }
+}
+
+static GemmPlan gemm_plan_bm(size_t k, const size_t *n, int count, size_t rows, int bm, bool tails) {
     GemmPlan p{};
-    p.nbs = (int)(n / 128);
     p.kbs = (int)(k / 128);
     p.bm = bm;
     p.mtiles = (int)((rows + p.bm - 1) / p.bm);
-    const int tiles = p.nbs * p.mtiles;
-    const int s = gemm_splits(p.kbs, tiles, p.bm);
-    if (p.bm < 128 && s == 1) return gemm_plan_bm(k, n, rows, 128);  // the 32/64-row tiles need a split
-    p.splits = s;
+    GemmSegment direct[kGemvMaxTargets], split[kGemvMaxTargets];
+    int nd = 0, ns = 0, nbs = 0;
+    bool many = count > 1;  // every matrix has a tile per CU and more: they share full rounds and one tail
+    for (int i = 0; i < count; ++i) {
+        nbs += (int)(n[i] / 128);
+        many = many && (int)(n[i] / 128) * p.mtiles > kGemmTargetWgs;
+    }
+    if (many) {
+        gemm_add(p, direct, nd, split, ns, 0, nbs, tails);
+    } else {  // each matrix as exl3_hip_mul_mat would split it: the same bits
+        for (int i = 0, nb0 = 0; i < count; ++i) {
+            gemm_add(p, direct, nd, split, ns, nb0, (int)(n[i] / 128), tails);
+            nb0 += (int)(n[i] / 128);
+        }
+    }
+    if (p.bm < 128 && nd) {  // the 32/64-row tiles need a split
+        if (count == 1) return gemm_plan_bm(k, n, count, rows, 128, tails);
+        return p;  // ok stays false
+    }
+    if (nd + ns > kGemmMaxSegments || (p.bm == 128 && nd && ns)) return p;  // (two different kernels)
+    int begin = 0, units = 0;
+    size_t blocks = 0;
+    for (int i = 0; i < nd + ns; ++i) {  // whole tiles first, they run longest
+        GemmSegment &g = p.grid.seg[i];
+        g = i < nd ? direct[i] : split[i - nd];
+        g.begin = begin;
+        begin += (g.tiles * g.splits + 7) & ~7;
+        g.unit0 = i < nd ? 0 : units;  // the reduction's ids fall into the split segments only
+        if (g.splits > 1) {
+            g.part0 = (unsigned)blocks;
+            blocks += (size_t)g.tiles * g.splits;
+            units += g.tiles * (p.bm / 16);
+            p.max_splits = g.splits > p.max_splits ? g.splits : p.max_splits;
+        }
+    }
+    p.grid.count = nd + ns;
+    p.grid.mtiles = p.mtiles;
+    p.grid.kbs = p.kbs;
+    p.workgroups = begin;
+    p.reduce_units = units;
     size_t off = kSharedPrefixBytes;  // the GEMM leaves the GEMV exchange alone
     p.xh_off = off;
-    off += ((size_t)p.mtiles * p.bm * k * 2 + 255) & ~(size_t)255;
+    p.xh_bytes = ((size_t)p.mtiles * p.bm * k * 2 + 255) & ~(size_t)255;
+    off += p.xh_bytes * count;
     p.partials_off = off;
-    if (s > 1) off += (size_t)tiles * s * p.bm * 128 * 2;  // fp16 partials
+    off += blocks * p.bm * 128 * 2;  // fp16 partials
     p.exps_off = off;
-    if (s > 1) off += ((size_t)tiles * s * (p.bm / 32) * 4 * 4 + 255) & ~(size_t)255;  // one per 32x32 block
+    off += (blocks * (p.bm / 32) * 4 * 4 + 255) & ~(size_t)255;  // one per 32x32 block
     p.bytes = (off + 255) & ~(size_t)255;
+    p.ok = true;
     return p;
 }
 
-GemmPlan gemm_plan(size_t k, size_t n, size_t rows) { return gemm_plan_bm(k, n, rows, gemm_tile_rows(rows)); }
+GemmPlan gemm_plan(size_t k, size_t n, size_t rows, bool tails) {
+    return gemm_plan_bm(k, &n, 1, rows, gemm_tile_rows(rows), tails);
+}
+GemmPlan gemm_plan_group(size_t k, const size_t *n, int count, size_t rows) {
+    return gemm_plan_bm(k, n, count, rows, gemm_tile_rows(rows), true);
+}
 
 // one tile class: kernel <RB, W> (NSG scheduling groups per k-step, XD activation
 // k-steps in flight) and its reduction
 template <int K, int CB, int RB, int W, int NSG, int XD, int CH>
-static void launch_gemm_tiles(const uint8_t *rec, size_t k, uint16_t *xh, size_t rows, void *y, int y_f16,
-                              size_t y_stride, uint8_t *ws, const GemmPlan &p, hipStream_t stream, const void *res,
-                              size_t res_stride) {
+static void launch_gemm_tiles(const GemvTargets &tg, const uint16_t *xh, size_t rows, int y_f16, uint8_t *ws,
+                              const GemmPlan &p, hipStream_t stream) {
     constexpr int WR = W / CH;  // the reduction sees the row waves
     static_assert(32 * RB * WR == 32 || 32 * RB * WR == 64 || 32 * RB * WR == 128 || 32 * RB * WR == 256 || 32 * RB * WR == 512,
                   "tile height");
-    const dim3 grid((unsigned)(p.mtiles * p.nbs * p.splits)), block(W * 64);
+    const dim3 grid((unsigned)p.workgroups), block(W * 64);
     uint16_t *part = (uint16_t *)(ws + p.partials_off);
     int *exps = (int *)(ws + p.exps_off);
-    const int nunits = p.mtiles * p.nbs * (p.bm / 16);  // reduction: one 4-wave workgroup per 16 rows of a tile
-    const int kq = p.kbs / p.splits, kr = p.kbs % p.splits;
-    gemm_kernel<K, CB, RB, W, NSG, XD, CH><<<grid, block, 0, stream>>>(
-        rec, p.kbs, p.nbs, p.mtiles, p.splits, kq, kr, xh, k, part, exps, y, y_f16, y_stride, (int)rows, res,
-        res_stride);
-    if (p.splits > 1)
-    {  // SB splits' loads in flight per batch: one batch for up to 16 splits (the
-       // 32-row tiles' 16: -0.4 to -0.6 us per call against two batches of 8)
-        if (p.splits > 8)
-            gemm_reduce_kernel<RB, WR, 16><<<dim3((unsigned)nunits), dim3(256), 0, stream>>>(
-                part, exps, p.splits, p.nbs, rec, K, p.kbs, y, y_f16, y_stride, (int)rows, nunits, res, res_stride);
-        else
-            gemm_reduce_kernel<RB, WR, 8><<<dim3((unsigned)nunits), dim3(256), 0, stream>>>(
-                part, exps, p.splits, p.nbs, rec, K, p.kbs, y, y_f16, y_stride, (int)rows, nunits, res, res_stride);
+    gemm_kernel<K, CB, RB, W, NSG, XD, CH><<<grid, block, 0, stream>>>(tg, p.grid, xh, p.xh_bytes / 2, part, exps,
+                                                                       y_f16, (int)rows);
+    if (p.reduce_units) {  // one 4-wave workgroup per 16 rows of a split tile
+        // SB splits' loads in flight per batch: one batch for up to 16 splits (the
+        // 32-row tiles' 16: -0.4 to -0.6 us per call against two batches of 8)
+        const dim3 units((unsigned)p.reduce_units);
+        GemmGrid gg = p.grid;
+        const bool one = tg.count == 1;  // at most one segment without a split before it
+        if (one) gg.seg[0] = gg.seg[gg.count - 1];
+        auto reduce = [&](auto sb, auto is_one) {
+            gemm_reduce_kernel<RB, WR, decltype(sb)::value, decltype(is_one)::value>
+                <<<units, dim3(256), 0, stream>>>(tg, gg, K, part, exps, y_f16, (int)rows);
+        };
+        typedef std::integral_constant<int, 16> S16;
+        typedef std::integral_constant<int, 8> S8;
+        if (p.max_splits > 8) one ? reduce(S16{}, std::true_type{}) : reduce(S16{}, std::false_type{});
+        else one ? reduce(S8{}, std::true_type{}) : reduce(S8{}, std::false_type{});
     }
 }
 
 template <int K, int CB>
-static void launch_gemm_kc(const uint8_t *rec, size_t k, uint16_t *xh, size_t rows, void *y, int y_f16,
-                           size_t y_stride, uint8_t *ws, const GemmPlan &p, hipStream_t stream, const void *res,
-                           size_t res_stride) {
+static void launch_gemm_kc(const GemvTargets &tg, const uint16_t *xh, size_t rows, int y_f16, uint8_t *ws,
+                           const GemmPlan &p, hipStream_t stream) {
     if (p.bm == 32)  // 4 waves: 4 column quarters (the plan gives it a split)
-        launch_gemm_tiles<K, CB, 1, 4, 0, 8, 4>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride);
+        launch_gemm_tiles<K, CB, 1, 4, 0, 8, 4>(tg, xh, rows, y_f16, ws, p, stream);
     else if (p.bm == 64)  // 8 waves: 2 row waves x 4 column quarters (the plan gives it a split)
-        launch_gemm_tiles<K, CB, 1, 8, 0, 8, 4>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride);
-    else if (p.bm == 128 && p.splits > 1)  // 8 waves: 4 row waves x 2 column halves, two waves per SIMD
-        launch_gemm_tiles<K, CB, 1, 8, 0, 8, 2>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride);
+        launch_gemm_tiles<K, CB, 1, 8, 0, 8, 4>(tg, xh, rows, y_f16, ws, p, stream);
+    else if (p.bm == 128 && p.reduce_units)  // 8 waves: 4 row waves x 2 column halves, two waves per SIMD
+        launch_gemm_tiles<K, CB, 1, 8, 0, 8, 2>(tg, xh, rows, y_f16, ws, p, stream);
     else if (p.bm == 128)
-        launch_gemm_tiles<K, CB, 1, 4, 8, 8, 1>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride);
+        launch_gemm_tiles<K, CB, 1, 4, 8, 8, 1>(tg, xh, rows, y_f16, ws, p, stream);
     else if (p.bm == 256)
-        launch_gemm_tiles<K, CB, 2, 4, 8, 8, 1>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride);
+        launch_gemm_tiles<K, CB, 2, 4, 8, 8, 1>(tg, xh, rows, y_f16, ws, p, stream);
     else  // 8 waves: no scheduling groups, four activation k-steps in flight (measured best at M = 512)
-        launch_gemm_tiles<K, CB, 2, 8, 0, 4, 1>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride);
+        launch_gemm_tiles<K, CB, 2, 8, 0, 4, 1>(tg, xh, rows, y_f16, ws, p, stream);
 }
 
 template <int K>
-static hipError_t launch_gemm_k(const void *records, int cb, size_t k, const void *x, int x_f16, size_t rows,
-                                size_t x_stride, void *y, int y_f16, size_t y_stride, uint8_t *ws, const GemmPlan &p,
-                                hipStream_t stream, const void *res, size_t res_stride) {
-    const uint8_t *rec = (const uint8_t *)records;
+static hipError_t launch_gemm_k(const GemvTargets &tg, int cb, const void *x, int x_f16, size_t rows, size_t x_stride,
+                                int y_f16, uint8_t *ws, const GemmPlan &p, hipStream_t stream) {
     uint16_t *xh = (uint16_t *)(ws + p.xh_off);
-    const int rows_padded = p.mtiles * p.bm;
-    gemm_xprep_kernel<<<dim3(p.kbs, rows_padded / 8), dim3(64), 0, stream>>>(rec, K, x, x_f16, x_stride, (int)rows,
-                                                                               p.kbs, xh);
+    const dim3 grid((unsigned)p.kbs, (unsigned)(p.mtiles * p.bm / 8), (unsigned)tg.count);
+    (tg.count == 1 ? gemm_xprep_kernel<true> : gemm_xprep_kernel<false>)<<<grid, dim3(64), 0, stream>>>(
+        tg, K, x, x_f16, x_stride, (int)rows, p.kbs, xh, p.xh_bytes / 2);
     switch (cb) {
-    case 0: launch_gemm_kc<K, 0>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride); break;
-    case 1: launch_gemm_kc<K, 1>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride); break;
-    default: launch_gemm_kc<K, 2>(rec, k, xh, rows, y, y_f16, y_stride, ws, p, stream, res, res_stride); break;
+    case 0: launch_gemm_kc<K, 0>(tg, xh, rows, y_f16, ws, p, stream); break;
+    case 1: launch_gemm_kc<K, 1>(tg, xh, rows, y_f16, ws, p, stream); break;
+    default: launch_gemm_kc<K, 2>(tg, xh, rows, y_f16, ws, p, stream); break;
     }
     return hipGetLastError();
 }
 
-hipError_t launch_gemm(const void *records, int bits, int cb, size_t k, size_t n, const void *x, int x_f16,
-                       size_t rows, size_t x_stride, void *y, int y_f16, size_t y_stride, void *workspace,
-                       const GemmPlan &p, hipStream_t stream, const void *res, size_t res_stride) {
-    (void)n;
+hipError_t launch_gemm_targets(const GemvTargets &tg, int bits, int cb, const void *x, int x_f16, size_t rows,
+                               size_t x_stride, int y_f16, void *workspace, const GemmPlan &p, hipStream_t stream) {
     uint8_t *ws = (uint8_t *)workspace;
     switch (bits) {
-    case 1: return launch_gemm_k<1>(records, cb, k, x, x_f16, rows, x_stride, y, y_f16, y_stride, ws, p, stream, res,
-                                       res_stride);
-    case 2: return launch_gemm_k<2>(records, cb, k, x, x_f16, rows, x_stride, y, y_f16, y_stride, ws, p, stream, res,
-                                       res_stride);
-    case 3: return launch_gemm_k<3>(records, cb, k, x, x_f16, rows, x_stride, y, y_f16, y_stride, ws, p, stream, res,
-                                       res_stride);
-    case 4: return launch_gemm_k<4>(records, cb, k, x, x_f16, rows, x_stride, y, y_f16, y_stride, ws, p, stream, res,
-                                       res_stride);
-    case 5: return launch_gemm_k<5>(records, cb, k, x, x_f16, rows, x_stride, y, y_f16, y_stride, ws, p, stream, res,
-                                       res_stride);
-    case 6: return launch_gemm_k<6>(records, cb, k, x, x_f16, rows, x_stride, y, y_f16, y_stride, ws, p, stream, res,
-                                       res_stride);
-    case 7: return launch_gemm_k<7>(records, cb, k, x, x_f16, rows, x_stride, y, y_f16, y_stride, ws, p, stream, res,
-                                       res_stride);
-    default: return launch_gemm_k<8>(records, cb, k, x, x_f16, rows, x_stride, y, y_f16, y_stride, ws, p, stream, res,
-                                       res_stride);
+    case 1: return launch_gemm_k<1>(tg, cb, x, x_f16, rows, x_stride, y_f16, ws, p, stream);
+    case 2: return launch_gemm_k<2>(tg, cb, x, x_f16, rows, x_stride, y_f16, ws, p, stream);
+    case 3: return launch_gemm_k<3>(tg, cb, x, x_f16, rows, x_stride, y_f16, ws, p, stream);
+    case 4: return launch_gemm_k<4>(tg, cb, x, x_f16, rows, x_stride, y_f16, ws, p, stream);
+    case 5: return launch_gemm_k<5>(tg, cb, x, x_f16, rows, x_stride, y_f16, ws, p, stream);
+    case 6: return launch_gemm_k<6>(tg, cb, x, x_f16, rows, x_stride, y_f16, ws, p, stream);
+    case 7: return launch_gemm_k<7>(tg, cb, x, x_f16, rows, x_stride, y_f16, ws, p, stream);
+    default: return launch_gemm_k<8>(tg, cb, x, x_f16, rows, x_stride, y_f16, ws, p, stream);
     }
 }
 

@@ -749,21 +749,6 @@ hipError_t launch_gemv_targets(const GemvTargets &tg, int bits, int cb, const vo
     }
 }
 
-hipError_t launch_gemv(const void *records, int bits, int cb, size_t k, size_t n, const void *x, int x_f16,
-                       size_t rows, size_t x_stride, void *y, int y_f16, size_t y_stride, void *workspace,
-                       const GemvPlan &p, hipStream_t stream, const void *res, size_t res_stride) {
-    (void)k;
-    GemvTargets tg{};
-    tg.records[0] = (const uint8_t *)records;
-    tg.y[0] = y;
-    tg.y_stride[0] = y_stride;
-    tg.res[0] = res;
-    tg.res_stride[0] = res_stride;
-    tg.nb_end[0] = (int)(n / 128);
-    tg.count = 1;
-    return launch_gemv_targets(tg, bits, cb, x, x_f16, rows, x_stride, y_f16, workspace, p, stream);
-}
-
 }  // namespace exl3k
 
 #ifdef EXL3_PHASE_STAMPS

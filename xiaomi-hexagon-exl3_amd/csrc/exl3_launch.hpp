@@ -57,7 +57,7 @@ int exchange_spin_limit();   // the wait budget of the split-K hand-off (polls p
 int exchange_drop_split();   // -1 unless a test dropped a split
 
 // Up to kGemvMaxTargets matrices that share k, the bit rate, the codebook and x,
-// served by one GEMV launch: column groups [nb_end[i-1], nb_end[i]) belong to
+// served by one GEMV or GEMM launch: column groups [nb_end[i-1], nb_end[i]) belong to
 // matrix i (records[i], output y[i] with row stride y_stride[i] elements).
 constexpr int kGemvMaxTargets = 4;
 struct GemvTargets {
@@ -87,9 +87,26 @@ struct GemvPlan {
     size_t partials_off, exchange_bytes, dummy_off, xpre_off, bytes;
     bool fits;  // the partials fit the exchange (else the call runs as a GEMM)
 };
+// One run of the GEMM's workgroups: the tiles tile0 .. tile0 + tiles - 1, tile t being
+// column group nb0 + t / mtiles (numbered over all targets) and m-tile t % mtiles, each
+// in `splits` k splits (split s has kq + (s < kr) records).
+struct GemmSegment {
+    int begin;           // first workgroup id, a multiple of 8
+    int nb0, tile0, tiles, splits, kq, kr;
+    unsigned part0;      // first (tile, split) partial block, when split
+    int unit0;           // first workgroup of the reduction, when split
+};
+constexpr int kGemmMaxSegments = 4;
+struct GemmGrid {
+    GemmSegment seg[kGemmMaxSegments];  // those without a split first
+    int count, mtiles, kbs;
+};
 struct GemmPlan {
-    int nbs, kbs, bm, mtiles, splits;  // bm: rows per workgroup tile (128, 256 or 512)
-    size_t xh_off, partials_off, exps_off, bytes;
+    bool ok;              // one launch can serve it (always, for one matrix)
+    int kbs, bm, mtiles;  // bm: rows per workgroup tile (32 .. 512)
+    int workgroups, reduce_units, max_splits;
+    GemmGrid grid;
+    size_t xh_off, xh_bytes, partials_off, exps_off, bytes;  // xh_bytes: activations of one target
 };
 
 GemvPlan gemv_plan(size_t k, size_t n, size_t rows);
@@ -98,19 +115,20 @@ bool gemv_serves(size_t k, size_t n, size_t rows);
 // the GEMV for one matrix: up to kGemvSingleMaxRows rows, and at 15..16 rows where
 // a workgroup preps at most kGemvSinglePrepBlocks (record, row) blocks
 bool gemv_serves_single(size_t k, size_t n, size_t rows);
-GemmPlan gemm_plan(size_t k, size_t n, size_t rows);
+// tails: the last round's tiles may be split where more tiles than CUs remain whole;
+// without, the plan (and its workspace) splits all tiles or none
+GemmPlan gemm_plan(size_t k, size_t n, size_t rows, bool tails);
+// the matrices of a grouped call in one launch: below a tile per CU each split as
+// gemm_plan splits it alone, above all together
+GemmPlan gemm_plan_group(size_t k, const size_t *n, int count, size_t rows);
 int gemm_tile_rows(size_t rows);
 
-// res (optional, y's dtype, row stride res_stride): y = res + layer(x), the sum
+// a target's res (optional, y's dtype, row stride res_stride): y = res + layer(x), the sum
 // rounded once; res may be y itself (same stride)
-hipError_t launch_gemv(const void *records, int bits, int cb, size_t k, size_t n, const void *x, int x_f16,
-                       size_t rows, size_t x_stride, void *y, int y_f16, size_t y_stride, void *workspace,
-                       const GemvPlan &plan, hipStream_t stream, const void *res = nullptr, size_t res_stride = 0);
 hipError_t launch_gemv_targets(const GemvTargets &targets, int bits, int cb, const void *x, int x_f16, size_t rows,
                                size_t x_stride, int y_f16, void *workspace, const GemvPlan &plan, hipStream_t stream);
-hipError_t launch_gemm(const void *records, int bits, int cb, size_t k, size_t n, const void *x, int x_f16,
-                       size_t rows, size_t x_stride, void *y, int y_f16, size_t y_stride, void *workspace,
-                       const GemmPlan &plan, hipStream_t stream, const void *res = nullptr, size_t res_stride = 0);
+hipError_t launch_gemm_targets(const GemvTargets &targets, int bits, int cb, const void *x, int x_f16, size_t rows,
+                               size_t x_stride, int y_f16, void *workspace, const GemmPlan &plan, hipStream_t stream);
 hipError_t launch_decode(const void *src, int records_layout, int bits, int cb, size_t k, size_t n,
                          size_t first, size_t count, uint16_t *out, hipStream_t stream);
 hipError_t launch_decode_batch(const DecodeBatch &batch, int records_layout, int bits, int cb, unsigned workgroups,
@@ -128,5 +146,9 @@ hipError_t launch_pack_records(const uint16_t *packed, const uint16_t *su, const
                                size_t n, void *records, hipStream_t stream);
 hipError_t launch_validate(const void *records, size_t nrecords, int bits, int *result, hipStream_t stream);
 hipError_t launch_zero(void *ptr, size_t bytes, hipStream_t stream);
+
+// The least workspace exl3_hip_mul_mat takes (exl3_api.cpp): plans without split tails.
+// exl3_hip_mul_mat_workspace_bytes reports what the fastest plans need.
+size_t mul_mat_least_workspace(size_t k, size_t n, size_t rows);
 
 }  // namespace exl3k
