@@ -102,9 +102,10 @@ constexpr size_t kGemvFragLds16 = 65536;  // the same for rows 9..16 (two workgr
 // runs one workgroup per CU.
 template <int K, int CB, int MODE>
 __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void gemv_kernel(
-    GemvTargets tg, int kbs, int splits, int kq, int kr, const void *__restrict__ x, int x_f16, size_t x_stride,
-    int rows, const uint8_t *__restrict__ dummy, uint32_t *__restrict__ partials, int y_f16,
-    const uint8_t *__restrict__ xpre, uint32_t *__restrict__ status, int spin_limit, int drop_split) {
+    GemvTargets tg, int kbs, int splits, int kq, int kr, const void *__restrict__ x_arg, int x_f16, size_t x_stride,
+    int rows, const uint8_t *__restrict__ dummy_arg, uint32_t *__restrict__ partials, int y_f16,
+    const uint8_t *__restrict__ xpre, uint32_t *__restrict__ status, int spin_limit, int drop_split,
+    uint32_t rows_inv) {
     constexpr bool TWO = MODE >= 1, HILO = MODE <= 1;
     constexpr int W = kGemvWaves;
     constexpr int P = W / 4;  // waves per column pair
@@ -134,27 +135,42 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
     if constexpr (MODE == 1) __builtin_amdgcn_s_setprio(1);
     const int kb0 = s * kq + (s < kr ? s : kr), kb1 = kb0 + kq + (s < kr ? 1 : 0);
     const int nkb = kb1 - kb0;
-    // the matrix of column group nb (targets share k, x and the bit rate)
-    int mi = 0;
-#pragma unroll
-    for (int i = 1; i < kGemvMaxTargets; ++i)
-        if (i < tg.count && nb >= tg.nb_end[i - 1]) mi = i;
-    const uint8_t *records = tg.records[0];
-    void *y = tg.y[0];
-    size_t y_stride = tg.y_stride[0];
-    const void *res = tg.res[0];
-    size_t res_stride = tg.res_stride[0];
-    int nbl = nb;  // column group within the matrix
-#pragma unroll
-    for (int i = 1; i < kGemvMaxTargets; ++i)
-        if (mi == i) {
-            records = tg.records[i];
-            y = tg.y[i];
-            y_stride = tg.y_stride[i];
-            res = tg.res[i];
-            res_stride = tg.res_stride[i];
-            nbl = nb - tg.nb_end[i - 1];
-        }
+    // the matrix of column group nb (targets share k, x and the bit rate).  The empty asm
+    // takes every argument at once, so that they arrive in one round of scalar loads; the
+    // compiler otherwise selects between the targets' argument addresses and loads again
+    // behind that
+    typedef const __attribute__((address_space(1))) uint8_t *global_bytes;  // stays global behind the asm
+    global_bytes rec0 = (global_bytes)tg.records[0], rec1 = (global_bytes)tg.records[1];
+    global_bytes rec2 = (global_bytes)tg.records[2], rec3 = (global_bytes)tg.records[3];
+    global_bytes xg = (global_bytes)x_arg, dg = (global_bytes)dummy_arg;
+    void *y0 = tg.y[0], *y1 = tg.y[1], *y2 = tg.y[2], *y3 = tg.y[3];
+    const void *q0 = tg.res[0], *q1 = tg.res[1], *q2 = tg.res[2], *q3 = tg.res[3];
+    size_t ys0 = tg.y_stride[0], ys1 = tg.y_stride[1], ys2 = tg.y_stride[2], ys3 = tg.y_stride[3];
+    size_t qs0 = tg.res_stride[0], qs1 = tg.res_stride[1], qs2 = tg.res_stride[2], qs3 = tg.res_stride[3];
+    int e0 = tg.nb_end[0], e1 = tg.nb_end[1], e2 = tg.nb_end[2], targets = tg.count;
+    asm volatile("" : "+s"(rec0), "+s"(rec1), "+s"(rec2), "+s"(rec3), "+s"(e0), "+s"(e1), "+s"(e2), "+s"(targets),
+                 "+s"(kbs), "+s"(xg), "+s"(x_stride), "+s"(x_f16), "+s"(dg));
+    const void *x = (const void *)xg;
+    const uint8_t *dummy = (const uint8_t *)dg;
+    int mi = 0, nbl = nb;  // nbl: column group within the matrix
+    global_bytes recs = rec0;
+    void *y = y0;
+    const void *res = q0;
+    size_t y_stride = ys0, res_stride = qs0;
+    auto take = [&](int i, int end, global_bytes r, void *yy, const void *q, size_t ys, size_t qs) {
+        const bool in = i < targets && nb >= end;
+        mi = in ? i : mi;
+        nbl = in ? nb - end : nbl;
+        recs = in ? r : recs;
+        y = in ? yy : y;
+        res = in ? q : res;
+        y_stride = in ? ys : y_stride;
+        res_stride = in ? qs : res_stride;
+    };
+    take(1, e0, rec1, y1, q1, ys1, qs1);
+    take(2, e1, rec2, y2, q2, ys2, qs2);
+    take(3, e2, rec3, y3, q3, ys3, qs3);
+    const uint8_t *records = (const uint8_t *)recs;
     const uint8_t *colgroup = records + (size_t)nbl * kbs * GB;
 
     // output scales for the epilogue (record (nb, 0), src/exl3-ggml.cpp:84-85)
@@ -188,6 +204,11 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
     // block (never stored), so the loads are straight-line code and all in
     // flight together.
     const int nblk = nkb * rows;
+    // blk / rows without a division (its expansion selects on vcc three times, 18 cycles
+    // each, ahead of the loads): rows_inv = ceil(2^16 / rows), exact while
+    // blk (rows - 1) < 2^16, and a workgroup has at most kGemvPrepMax W blocks
+    auto by_rows = [&](int blk) { return (int)(((uint32_t)blk * rows_inv) >> 16); };
+    static_assert(kGemvPrepMax * kGemvWaves * 16 <= 1 << 16, "by_rows");
     auto prologue = [&](auto nq_c, auto is_f16) {
         constexpr int NQ = decltype(nq_c)::value;
         constexpr bool XF16 = decltype(is_f16)::value;
@@ -197,7 +218,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
         for (int q = 0; q < NQ; ++q) {
             const int bu = (4 * q + g) * W + wave;
             const int blk = bu < nblk ? bu : nblk - 1;
-            const int kbl = blk / rows, r = blk - kbl * rows;
+            const int kbl = by_rows(blk), r = blk - kbl * rows;
             const int kb = kb0 + kbl;
             sr[q] = *(const uint4 *)(records + (size_t)kb * GB + 2048 * K + 16 * pi);  // record (0, kb): su
             const size_t xi = (size_t)r * x_stride + (size_t)kb * 128 + 8 * pi;
@@ -262,11 +283,11 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
                     lane_stage(std::integral_constant<int, 4>{});
                     lane_stage(std::integral_constant<int, 8>{});
                 }
-                const float scale = (__builtin_popcount(pi & 15) & 1) ? -0.08838834764831844055f
-                                                                       : 0.08838834764831844055f;
+                const float scale = __uint_as_float(__float_as_uint(0.08838834764831844055f) ^
+                                                    ((uint32_t)__builtin_popcount(pi & 15) << 31));
                 const int blk = (4 * q + g) * W + wave;
                 if (blk < nblk) {
-                    const int kbl = blk / rows, r = blk - kbl * rows;
+                    const int kbl = by_rows(blk), r = blk - kbl * rows;
                     h8 hi, lo;
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
@@ -292,7 +313,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
     auto prologue_one = [&](auto is_f16) {
         constexpr bool XF16 = decltype(is_f16)::value;
         const int blk = wave < nblk ? wave : nblk - 1;
-        const int kbl = blk / rows, r = blk - kbl * rows;
+        const int kbl = by_rows(blk), r = blk - kbl * rows;
         const int kb = kb0 + kbl;
         const uint32_t ps = ((const uint32_t *)(records + (size_t)kb * GB + 2048 * K))[lane];  // su pair
         const size_t xi = (size_t)r * x_stride + (size_t)kb * 128 + 2 * lane;
@@ -363,7 +384,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
     const int mrow = r1 < rows ? r1 : rows - 1, mrow2 = r2 < rows ? r2 : rows - 1;  // TWO: the second block
     const int boff = (HILO ? (g * 2 + hl) * rows + mrow : g * rows + mrow) * 16;
     const int boff2 = (HILO ? (g * 2 + hl) * rows + mrow2 : g * rows + mrow2) * 16;
-    const bool first_chunk = j == 0;
+    uint32_t first_chunk = j == 0 ? ~0u : 0u;
+    asm("" : "+v"(first_chunk));  // a mask: the select below is then v_bfi_b32, not v_cndmask_b32 on vcc (18 cycles)
     f4 acc1 = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
     f4 acc3 = {0.f, 0.f, 0.f, 0.f}, acc4 = {0.f, 0.f, 0.f, 0.f};  // TWO: acc1 / acc2 of rows 8..15
     auto mac = [&](int i, const uint32_t (&w)[K]) {
@@ -371,7 +393,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
         const uint32_t p1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)w[K - 1], 0x121, 0xF, 0xF, false);  // row_ror:1
         const uint32_t p9 = (uint32_t)__builtin_amdgcn_mov_dpp((int)w[K - 1], 0x129, 0xF, 0xF, false);  // row_ror:9
         u4 fr[4];
-        decode_chunk<K, CB>(w, first_chunk ? p9 : p1, fr);
+        decode_chunk<K, CB>(w, (first_chunk & p9) | (~first_chunk & p1), fr);
         const uint8_t *bp = frag + (size_t)group_q(i) * 2 * blk_bytes + boff;
         const h8 blo = *(const h8 *)bp, bhi = *(const h8 *)(bp + blk_bytes);
         acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(bitcast<h8>(fr[0]), blo, acc1, 0, 0, 0);
@@ -413,13 +435,13 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
         const int n = 4 * g + e;
         if (m < rows) {
             float *rp = red + part * nval + m * 128 + 32 * cp;
-            rp[n < 8 ? n : 8 + n] = acc1[e];
-            rp[n < 8 ? 8 + n : 16 + n] = acc2[e];
+            rp[n + (n & 8)] = acc1[e];
+            rp[8 + n + (n & 8)] = acc2[e];
         }
         if (16 + m < rows) {
             float *rp = red + part * nval + (16 + m) * 128 + 32 * cp;
-            rp[n < 8 ? n : 8 + n] = acc3[e];
-            rp[n < 8 ? 8 + n : 16 + n] = acc4[e];
+            rp[n + (n & 8)] = acc3[e];
+            rp[8 + n + (n & 8)] = acc4[e];
         }
     }
 #pragma unroll
@@ -429,16 +451,16 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
         const float o2 = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc2[e]), 0x108, 0xF, 0xF, true));
         if (m < 8 && m < rows) {
             float *rp = red + part * nval + m * 128 + 32 * cp;
-            rp[n < 8 ? n : 8 + n] = acc1[e] + o1;
-            rp[n < 8 ? 8 + n : 16 + n] = acc2[e] + o2;
+            rp[n + (n & 8)] = acc1[e] + o1;
+            rp[8 + n + (n & 8)] = acc2[e] + o2;
         }
         if constexpr (TWO) {
             const float o3 = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc3[e]), 0x108, 0xF, 0xF, true));
             const float o4 = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc4[e]), 0x108, 0xF, 0xF, true));
             if (m < 8 && 8 + m < rows) {
                 float *rp = red + part * nval + (8 + m) * 128 + 32 * cp;
-                rp[n < 8 ? n : 8 + n] = acc3[e] + o3;
-                rp[n < 8 ? 8 + n : 16 + n] = acc4[e] + o4;
+                rp[n + (n & 8)] = acc3[e] + o3;
+                rp[8 + n + (n & 8)] = acc4[e] + o4;
             }
         }
     }
@@ -552,11 +574,12 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
                 }
 #pragma unroll
                 for (int jb = 0; jb < B; ++jb)
-                    if (base + jb < nsp) {  // a word that never filled: a loud result, not a hang
-                        a0 += v0[jb] && !poisoned ? exchange_value(v0[jb]) : __builtin_nanf("");
-                        a1 += v1[jb] && !poisoned ? exchange_value(v1[jb]) : __builtin_nanf("");
+                    if (base + jb < nsp) {  // a word that never filled (zero) reads as NaN: a loud result, not a hang
+                        a0 += exchange_value(v0[jb]);
+                        a1 += exchange_value(v1[jb]);
                     }
             }
+            if (poisoned) a0 = a1 = __builtin_nanf("");
             if (rr == 0) stamps.mark(4);
             finish_row(rr, a0 + own[rr * 128 + lane], a1 + own[rr * 128 + lane + 64]);
             if (rr == 0) stamps.mark(5);
@@ -705,21 +728,22 @@ static hipError_t launch_gemv_kc(const GemvTargets &tg, const void *x, int x_f16
     uint32_t *status = (uint32_t *)(ws + kStatusOffset);
     const int spin_limit = exchange_spin_limit();
     const int drop_split = exchange_drop_split();
+    const uint32_t rows_inv = (uint32_t)((65536 + rows - 1) / rows);
     if (rows > 16) {
         uint16_t *xp = (uint16_t *)(ws + p.xpre_off);
         gemv_xprep_kernel<<<dim3((unsigned)((rows + 3) / 4), (unsigned)p.kbs, (unsigned)tg.count), dim3(256), 0,
                             stream>>>(tg, K, x, x_f16, x_stride, (int)rows, p.kbs, xp);
         gemv_kernel<K, CB, 2><<<grid, block, lds, stream>>>(tg, p.kbs, p.splits, kq, kr, x, x_f16, x_stride,
                                                             (int)rows, ws + p.dummy_off, part, y_f16,
-                                                            (const uint8_t *)xp, status, spin_limit, drop_split);
+                                                            (const uint8_t *)xp, status, spin_limit, drop_split, rows_inv);
     } else if (rows > 8) {
         gemv_kernel<K, CB, 1><<<grid, block, lds, stream>>>(tg, p.kbs, p.splits, kq, kr, x, x_f16, x_stride,
                                                             (int)rows, ws + p.dummy_off, part, y_f16, nullptr,
-                                                            status, spin_limit, drop_split);
+                                                            status, spin_limit, drop_split, rows_inv);
     } else {
         gemv_kernel<K, CB, 0><<<grid, block, lds, stream>>>(tg, p.kbs, p.splits, kq, kr, x, x_f16, x_stride,
                                                             (int)rows, ws + p.dummy_off, part, y_f16, nullptr,
-                                                            status, spin_limit, drop_split);
+                                                            status, spin_limit, drop_split, rows_inv);
     }
     return hipGetLastError();
 }

@@ -57,7 +57,7 @@ constexpr int kExchangeSpinLimit = 1 << 20;  // polls per wave of the summing wo
 // 0xffffffff) is stored as 1, which reads back as the NaN 0xfffffffe
 __device__ __forceinline__ uint32_t exchange_bits(float v) {
     const uint32_t c = ~__float_as_uint(v);
-    return c ? c : 1u;
+    return c > 1u ? c : 1u;  // v_max_u32
 }
 __device__ __forceinline__ float exchange_value(uint32_t w) { return __uint_as_float(~w); }
 __device__ __forceinline__ void store_exchange(uint32_t *p, float v) {
