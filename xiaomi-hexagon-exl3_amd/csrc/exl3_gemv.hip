@@ -28,10 +28,9 @@ namespace exl3k {
 //      All activation loads of a wave are in flight together.
 //   2. weight stream: lane l = 16 g + i loads chunk i % 8 (K contiguous words)
 //      of tile (4 r4 + g, 2 c2 + i / 8): one K-word load per lane and group,
-//      DEPTH groups in flight, all issued after the prep barrier: weight loads
-//      issued earlier delay the activation loads of the other workgroups behind
-//      them (measured: 3 groups before the barrier cost 4 % at k = 14336, all 8
-//      cost 11 %), and the prep is on every workgroup's critical path.
+//      DEPTH groups in flight, at most two of them issued before the prep barrier
+//      (EARLY): weight loads delay the activation loads of the other workgroups
+//      behind them, and the prep is on every workgroup's critical path.
 //   3. a lane decodes its chunk's 32 weights in registers (the first states
 //      reach into the previous chunk's last word, taken from the neighbouring
 //      lane with DPP) into four MFMA A fragments (rows 0-7 / 8-15 of its tile row
@@ -189,6 +188,13 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
                            : dummy + lane_off;
     };
     uint32_t buf[D][K];
+    // Ring slots issued before the prep barrier.  Two in the prep of more than one block per
+    // wave (against one: 4 layers of hidden 4096 at 4 rows 245.9 -> 240.4 us, of hidden 2048
+    // at 16 rows 195.3 -> 190.8; four lose 3 to 8 %).  In the short one-block prep two from 5
+    // bits on (k = 4096, n = 14336 at 6 bits 16.10 -> 15.28 us), none below, where they delay
+    // the activations of the other workgroups (k = 14336, n = 4096 at 4 bits 12.67 -> 12.86).
+    constexpr int EARLY = 2;
+    constexpr bool kEarlyOne = K >= 5;
 
     // 1-2. prep: xh = H128(x[r] su) per (kb, row) block of the workgroup, as
     // fp16 hi = rn(xh) and lo = rn(xh - hi) into the B fragments.  Unit q of
@@ -226,10 +232,10 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
             if constexpr (XF16) __builtin_memcpy(&xr[q][0], (const uint16_t *)x + xi, 16);
             else __builtin_memcpy(&xr[q][0], (const float *)x + xi, 32);
         }
-        // the first weight-ring slot right behind the activation loads: its
-        // latency then passes under this prep's H128 work (the one-block prep
-        // below is too short for that and issues it after the barrier)
-        load_chunk<K>(group_src(0), buf[0]);
+        // the first weight-ring slots right behind the activation loads: their
+        // latency then passes under this prep's H128 work
+#pragma unroll
+        for (int d = 0; d < EARLY; ++d) load_chunk<K>(group_src(d), buf[d]);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
             if (4 * q * W + wave < nblk) {  // uniform in the wave: the DPP stages see every lane
@@ -325,6 +331,10 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
             a = ((const float *)x)[xi];
             b = ((const float *)x)[xi + 1];
         }
+        if constexpr (kEarlyOne) {
+#pragma unroll
+            for (int d = 0; d < EARLY; ++d) load_chunk<K>(group_src(d), buf[d]);
+        }
         if (wave < nblk) {
             a *= half_bits_to_float((uint16_t)(ps & 0xffffu));
             b *= half_bits_to_float((uint16_t)(ps >> 16));
@@ -372,9 +382,12 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
     __syncthreads();
     stamps.mark(1);
     if constexpr (MODE == 1) __builtin_amdgcn_s_setprio(0);
-    if (MODE == 2 || nblk <= W) load_chunk<K>(group_src(0), buf[0]);  // not issued by the prep
+    if (MODE == 2 || (!kEarlyOne && nblk <= W)) {  // not issued by the prep
 #pragma unroll
-    for (int d = 1; d < D; ++d) load_chunk<K>(group_src(d), buf[d]);
+        for (int d = 0; d < EARLY; ++d) load_chunk<K>(group_src(d), buf[d]);
+    }
+#pragma unroll
+    for (int d = EARLY; d < D; ++d) load_chunk<K>(group_src(d), buf[d]);
 
     // 4. decode + MFMA.  B operand lane l: m = l % 16 -> (hl, row) = (m / 8, m % 8),
     // k group l / 16; rows >= `rows` read the last row (their columns are discarded)
