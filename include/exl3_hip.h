@@ -342,11 +342,11 @@ exl3_status exl3_hip_pack_records(const uint16_t *packed, const uint16_t *su, co
 
 /* The DSP service's layer exl3_iface_matmul (src/hexagon/exl3_service.c:265-305,
  * IDL src/hexagon/exl3_iface.idl:13-15): y = x . diag(su) H W_hat H diag(sv) on the
- * upstream tile layout with separate su / sv vectors, fp32 in and out.  One call packs
- * the tiles and scales into group records inside the workspace (exl3_hip_pack_records)
- * and runs exl3_hip_mul_mat on them, so the weights are decoded once per call, as the
- * service decodes them; callers that reuse the weights pack once and call
- * exl3_hip_mul_mat instead.
+ * upstream tile layout with separate su / sv vectors, fp32 in and out.  Up to the row
+ * counts of exl3_hip_mul_mat's GEMV the kernel reads the tiles and scales as they are;
+ * above, one call packs them into group records inside the workspace
+ * (exl3_hip_pack_records) and runs exl3_hip_mul_mat on them (the same bits either way).
+ * Callers that reuse the weights at many rows pack once and call exl3_hip_mul_mat.
  *   packed      device, [k/16][n/16][16*bits] u16 = k*n*bits/8 bytes, 16-byte aligned
  *   suh, svh    device fp16 su[k] and sv[n], 16-byte aligned
  *   x, y        device fp32, batch x k and batch x n, dense rows (the service's layout)

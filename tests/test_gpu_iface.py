@@ -62,3 +62,24 @@ def test_iface_matmul_caller_workspace_repeated_calls(amd, oracle):
     small = ws[: ws.numel() - 1]
     with pytest.raises(amd.Exl3Error):
         amd.iface_matmul(pd, sud, svd, torch.zeros((8, k), device="cuda"), bits, k, n, workspace=small)
+
+
+@pytest.mark.parametrize("bits", range(1, 9))
+@pytest.mark.parametrize("k,n", [(128, 128), (640, 384), (2048, 256), (4224, 128)])
+def test_iface_reads_tiles_like_records(amd, bits, k, n):
+    """Every rate, one and many records per workgroup, odd record counts, the row counts around
+    the kernel's row modes and the row count that packs records instead: mul_mat's bits on the
+    packed records of the same weights."""
+    import torch
+    p, su, sv = upstream(650 + bits, k, n, bits)
+    pd, sud, svd = dev(p), dev(su.view(np.uint16)), dev(sv.view(np.uint16))
+    rec = amd.pack_records(pd, sud, svd, bits, k, n)
+    cb = bits % 3
+    print(f"  iface tiles k={k} n={n} bits={bits} cb={cb}", flush=True)
+    for rows in (1, 2, 7, 8, 9, 14, 15, 16, 17):
+        x = torch.from_numpy(synth.activations(660 + rows, rows, k).astype(np.float32)).cuda()
+        ws = amd.new_iface_workspace(bits, k, n, rows)
+        y = amd.iface_matmul(pd, sud, svd, x, bits, k, n, codebook=cb, workspace=ws)
+        again = amd.iface_matmul(pd, sud, svd, x, bits, k, n, codebook=cb, workspace=ws)
+        want = amd.mul_mat(rec, bits, k, n, x, codebook=cb, out_dtype=torch.float32)
+        assert torch.equal(y, want) and torch.equal(again, want), rows

@@ -627,6 +627,12 @@ exl3_status exl3_hip_iface_matmul(unsigned bits, unsigned codebook, size_t k, si
     const size_t need = least + (want - iface_records_offset(k, n, batch, true));
     exl3_status st = call_workspace(need, [&] { return want; }, stream, &workspace, &workspace_bytes);
     if (st != EXL3_OK) return st;
+    // the GEMV reads the tiles as they are (2048 x 6144, 5 bits, batch 8: 15.0 -> 10.3 us per
+    // call against packing records first); the GEMM, which reads each weight once per row
+    // tile too but decodes from whole records, gets them packed
+    if (exl3k::gemv_serves_single(k, n, batch))
+        return from_hip(exl3k::launch_gemv_tiles(packed, suh, svh, (int)bits, (int)codebook, x, batch, y, n, workspace,
+                                                 exl3k::gemv_plan(k, n, batch), stream));
     const size_t roff = workspace_bytes < want ? least : iface_records_offset(k, n, batch, true);
     void *records = (uint8_t *)workspace + roff;
     st = exl3_hip_pack_records(packed, suh, svh, bits, k, n, records, stream);

@@ -99,7 +99,10 @@ constexpr size_t kGemvFragLds16 = 65536;  // the same for rows 9..16 (two workgr
 // amdgpu_waves_per_eu(4): two workgroups per CU.  Without it the compiler places
 // the VGPR that holds spilled SGPRs (rows 17..32) at v222, and the kernel then
 // runs one workgroup per CU.
-template <int K, int CB, int MODE>
+// TILES (exl3_hip_iface_matmul): the weights are upstream tiles [k / 16][n / 16] instead
+// of group records, target 0's `records` the tiles, target 1's su and target 2's sv; x is
+// binary32.  A group's lanes read the same 64 chunks, its four tile rows 2 n K bytes apart.
+template <int K, int CB, int MODE, bool TILES = false>
 __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void gemv_kernel(
     GemvTargets tg, int kbs, int splits, int kq, int kr, const void *__restrict__ x_arg, int x_f16, size_t x_stride,
     int rows, const uint8_t *__restrict__ dummy_arg, uint32_t *__restrict__ partials, int y_f16,
@@ -166,25 +169,36 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
         y_stride = in ? ys : y_stride;
         res_stride = in ? qs : res_stride;
     };
-    take(1, e0, rec1, y1, q1, ys1, qs1);
-    take(2, e1, rec2, y2, q2, ys2, qs2);
-    take(3, e2, rec3, y3, q3, ys3, qs3);
+    if constexpr (!TILES) {
+        take(1, e0, rec1, y1, q1, ys1, qs1);
+        take(2, e1, rec2, y2, q2, ys2, qs2);
+        take(3, e2, rec3, y3, q3, ys3, qs3);
+    }
     const uint8_t *records = (const uint8_t *)recs;
-    const uint8_t *colgroup = records + (size_t)nbl * kbs * GB;
+    const uint32_t tile_row = gridDim.x * 256u * K;  // TILES: bytes of one tile row
+    const uint8_t *colgroup = records + (TILES ? (size_t)nbl * 256 * K : (size_t)nbl * kbs * GB);
+    // su of record (0, kb)
+    auto su_of = [&](int kb) {
+        return TILES ? (const uint8_t *)rec1 + (size_t)kb * 256 : records + (size_t)kb * GB + 2048 * K;
+    };
 
     // output scales for the epilogue (record (nb, 0), src/exl3-ggml.cpp:84-85)
-    const uint16_t *svp = (const uint16_t *)(colgroup + 2048 * K + 256);
+    const uint16_t *svp =
+        (const uint16_t *)(TILES ? (const uint8_t *)rec2 + (size_t)nbl * 256 : colgroup + 2048 * K + 256);
 
     // weight stream: this wave's groups are q = part + P i; issues past its
     // last group read the workspace's dummy region, so every issue is
     // unconditional and the compiler's wait counts stay exact
     const int g = lane >> 4, li = lane & 15, j = li & 7;
-    const uint32_t lane_off = (uint32_t)(((8 * g + 2 * cp + (li >> 3)) * 32 + 4 * j) * K);
+    const uint32_t lane_off = TILES ? g * tile_row + (uint32_t)(((2 * cp + (li >> 3)) * 32 + 4 * j) * K)
+                                    : (uint32_t)(((8 * g + 2 * cp + (li >> 3)) * 32 + 4 * j) * K);
     const int ngroups = (2 * nkb - part + P - 1) / P;
     auto group_q = [&](int i) { return part + P * i; };
     auto group_src = [&](int i) -> const uint8_t * {
         const int q = group_q(i);
-        return i < ngroups ? colgroup + (size_t)(kb0 + (q >> 1)) * GB + (size_t)(q & 1) * 1024 * K + lane_off
+        if constexpr (TILES)  // past the last group: the last one again (the dummy region is too small for the pitch)
+            return colgroup + (size_t)(8 * kb0 + 4 * (i < ngroups ? q : group_q(0))) * tile_row + lane_off;
+        else return i < ngroups ? colgroup + (size_t)(kb0 + (q >> 1)) * GB + (size_t)(q & 1) * 1024 * K + lane_off
                            : dummy + lane_off;
     };
     uint32_t buf[D][K];
@@ -226,7 +240,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
             const int blk = bu < nblk ? bu : nblk - 1;
             const int kbl = by_rows(blk), r = blk - kbl * rows;
             const int kb = kb0 + kbl;
-            sr[q] = *(const uint4 *)(records + (size_t)kb * GB + 2048 * K + 16 * pi);  // record (0, kb): su
+            sr[q] = *(const uint4 *)(su_of(kb) + 16 * pi);
             const size_t xi = (size_t)r * x_stride + (size_t)kb * 128 + 8 * pi;
             // element alignment only (any row stride): the compiler emits unaligned vector loads
             if constexpr (XF16) __builtin_memcpy(&xr[q][0], (const uint16_t *)x + xi, 16);
@@ -321,7 +335,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
         const int blk = wave < nblk ? wave : nblk - 1;
         const int kbl = by_rows(blk), r = blk - kbl * rows;
         const int kb = kb0 + kbl;
-        const uint32_t ps = ((const uint32_t *)(records + (size_t)kb * GB + 2048 * K))[lane];  // su pair
+        const uint32_t ps = ((const uint32_t *)su_of(kb))[lane];  // su pair
         const size_t xi = (size_t)r * x_stride + (size_t)kb * 128 + 2 * lane;
         float a, b;
         if constexpr (XF16) {
@@ -375,7 +389,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
             if (o < nbytes) *(u4 *)(frag + o) = cv[c];
         }
     } else {
-        if (x_f16) prologue_x(std::true_type{});
+        if constexpr (TILES) prologue_x(std::false_type{});
+        else if (x_f16) prologue_x(std::true_type{});
         else prologue_x(std::false_type{});
     }
     const float sv0 = half_bits_to_float(svp[lane]), sv1 = half_bits_to_float(svp[lane + 64]);
@@ -759,6 +774,52 @@ static hipError_t launch_gemv_kc(const GemvTargets &tg, const void *x, int x_f16
                                                             status, spin_limit, drop_split, rows_inv);
     }
     return hipGetLastError();
+}
+
+template <int K, int CB>
+static hipError_t launch_gemv_tiles_kc(const GemvTargets &tg, const float *x, size_t rows, uint8_t *ws,
+                                       const GemvPlan &p, hipStream_t stream) {
+    const size_t lds = gemv_lds_bytes(p.nkw, rows);
+    const dim3 grid((unsigned)p.nbs, (unsigned)p.splits), block(kGemvWaves * 64);
+    (rows > 8 ? gemv_kernel<K, CB, 1, true> : gemv_kernel<K, CB, 0, true>)<<<grid, block, lds, stream>>>(
+        tg, p.kbs, p.splits, p.kbs / p.splits, p.kbs % p.splits, x, 0, (size_t)p.kbs * 128, (int)rows,
+        ws + p.dummy_off, (uint32_t *)(ws + p.partials_off), 0, nullptr, (uint32_t *)(ws + kStatusOffset),
+        exchange_spin_limit(), exchange_drop_split(), (uint32_t)((65536 + rows - 1) / rows));
+    return hipGetLastError();
+}
+
+template <int K>
+static hipError_t launch_gemv_tiles_k(const GemvTargets &tg, int cb, const float *x, size_t rows, uint8_t *ws,
+                                      const GemvPlan &p, hipStream_t stream) {
+    switch (cb) {
+    case 0: return launch_gemv_tiles_kc<K, 0>(tg, x, rows, ws, p, stream);
+    case 1: return launch_gemv_tiles_kc<K, 1>(tg, x, rows, ws, p, stream);
+    default: return launch_gemv_tiles_kc<K, 2>(tg, x, rows, ws, p, stream);
+    }
+}
+
+hipError_t launch_gemv_tiles(const uint16_t *tiles, const uint16_t *su, const uint16_t *sv, int bits, int cb,
+                             const float *x, size_t rows, float *y, size_t n, void *workspace, const GemvPlan &p,
+                             hipStream_t stream) {
+    GemvTargets tg{};
+    tg.records[0] = (const uint8_t *)tiles;
+    tg.records[1] = (const uint8_t *)su;
+    tg.records[2] = (const uint8_t *)sv;
+    tg.y[0] = y;
+    tg.y_stride[0] = n;
+    tg.nb_end[0] = p.nbs;
+    tg.count = 1;
+    uint8_t *ws = (uint8_t *)workspace;
+    switch (bits) {
+    case 1: return launch_gemv_tiles_k<1>(tg, cb, x, rows, ws, p, stream);
+    case 2: return launch_gemv_tiles_k<2>(tg, cb, x, rows, ws, p, stream);
+    case 3: return launch_gemv_tiles_k<3>(tg, cb, x, rows, ws, p, stream);
+    case 4: return launch_gemv_tiles_k<4>(tg, cb, x, rows, ws, p, stream);
+    case 5: return launch_gemv_tiles_k<5>(tg, cb, x, rows, ws, p, stream);
+    case 6: return launch_gemv_tiles_k<6>(tg, cb, x, rows, ws, p, stream);
+    case 7: return launch_gemv_tiles_k<7>(tg, cb, x, rows, ws, p, stream);
+    default: return launch_gemv_tiles_k<8>(tg, cb, x, rows, ws, p, stream);
+    }
 }
 
 template <int K>

@@ -127,6 +127,10 @@ int gemm_tile_rows(size_t rows);
 // rounded once; res may be y itself (same stride)
 hipError_t launch_gemv_targets(const GemvTargets &targets, int bits, int cb, const void *x, int x_f16, size_t rows,
                                size_t x_stride, int y_f16, void *workspace, const GemvPlan &plan, hipStream_t stream);
+// the GEMV on upstream tiles with separate su and sv (dense binary32 x and y), rows <= 16
+hipError_t launch_gemv_tiles(const uint16_t *tiles, const uint16_t *su, const uint16_t *sv, int bits, int cb,
+                             const float *x, size_t rows, float *y, size_t n, void *workspace, const GemvPlan &plan,
+                             hipStream_t stream);
 hipError_t launch_gemm_targets(const GemvTargets &targets, int bits, int cb, const void *x, int x_f16, size_t rows,
                                size_t x_stride, int y_f16, void *workspace, const GemmPlan &plan, hipStream_t stream);
 hipError_t launch_decode(const void *src, int records_layout, int bits, int cb, size_t k, size_t n,
