@@ -205,3 +205,33 @@ def test_reconstruct_wave_layout(amd, oracle, bits, cb, records):
         got = amd.reconstruct(src, bits, k, n, su=su_t, sv=sv_t, codebook=cb, layout=layout, first=first, count=count,
                               out=out)
         assert np.array_equal(host_u16(got), want.view(np.uint16)), (bits, cb, shift)
+
+
+@pytest.mark.parametrize("records", [False, True])
+def test_decode_batch_mixed_rates_one_launch(amd, oracle, records):
+    """All eight rates in one call, more matrices than one launch takes, widths of one tile, of
+    part of a wave's 128 columns and of several, one to many tile rows: the oracle's bits, and
+    nothing written next to an output."""
+    import torch
+    for cb in range(3):
+        items, want, raws = [], [], []
+        shapes = [(128, 128), (256, 384), (128, 1152)] if records else [(16, 16), (48, 144), (16, 400), (272, 128),
+                                                                        (160, 1040)]
+        for i in range(40):
+            bits, (k, n) = 1 + (i * 5) % 8, shapes[i % len(shapes)]
+            p = synth.packed_tiles(3000 + 40 * cb + i, k, n, bits)
+            if records:
+                su, sv = synth.layer_scales(3000 + i, k, n)
+                src = dev(synth.pack_records(p, su, sv, bits).view(np.uint8))
+            else:
+                src = dev(p)
+            raw = torch.full((k * n + 16,), 0x5A5A, dtype=torch.int16, device="cuda")
+            raws.append(raw)
+            items.append((src, bits, k, n, raw[8: 8 + k * n].view(k, n)))
+            want.append(oracle.decode_inner(p, k, n, bits, cb))
+        print(f"  decode batch cb={cb} records={records}", flush=True)
+        outs = amd.decode_batch(items, codebook=cb,
+                                layout=amd.LAYOUT_RECORDS if records else amd.LAYOUT_UPSTREAM_TILES)
+        for (_, bits, k, n, _), got, ref, raw in zip(items, outs, want, raws):
+            assert np.array_equal(host_u16(got).reshape(k, n), ref.reshape(k, n)), (bits, k, n)
+            assert bool((raw[:8] == 0x5A5A).all()) and bool((raw[-8:] == 0x5A5A).all())

@@ -507,38 +507,36 @@ exl3_status exl3_hip_decode_batch(const exl3_decode_desc *descs, size_t count, e
             !valid_matrix(d.k, d.n, mult) || (d.k / 16) * ((d.n / 16 + 15) / 16) > (size_t)0x7fffffff)
             return EXL3_INVAL_PARAMS;
     }
-    // one launch per (rate, up to kDecodeBatchMax matrices); matrices keep their order within a rate
+    // one launch per kDecodeBatchMax matrices
     const int rl = layout == EXL3_LAYOUT_RECORDS;
-    for (unsigned bits = 1; bits <= 8; ++bits) {
-        exl3k::DecodeBatch b{};
-        size_t wgs = 0;
-        auto flush = [&]() -> exl3_status {
-            if (!b.count) return EXL3_OK;
-            const hipError_t e = exl3k::launch_decode_batch(b, rl, (int)bits, (int)codebook, (unsigned)wgs, stream);
-            b = exl3k::DecodeBatch{};
-            wgs = 0;
-            return from_hip(e);
-        };
-        for (size_t i = 0; i < count; ++i) {
-            const exl3_decode_desc &d = descs[i];
-            if (d.bits != bits) continue;
-            const size_t mwgs = ((d.k / 16) * ((d.n / 16 + 15) / 16) + exl3k::kDecodeBlocksPerWg - 1) / exl3k::kDecodeBlocksPerWg;
-            if (b.count == exl3k::kDecodeBatchMax || wgs + mwgs > (size_t)0x7fffffff) {
-                const exl3_status st = flush();
-                if (st != EXL3_OK) return st;
-            }
-            b.src[b.count] = d.src;
-            b.out[b.count] = d.out;
-            b.k[b.count] = d.k;
-            b.n[b.count] = d.n;
-            b.wg_begin[b.count] = (unsigned)wgs;
-            ++b.count;
-            wgs += mwgs;
+    exl3k::DecodeBatch b{};
+    size_t wgs = 0;
+    auto flush = [&]() -> exl3_status {
+        if (!b.count) return EXL3_OK;
+        const hipError_t e = exl3k::launch_decode_batch(b, rl, (int)codebook, (unsigned)wgs, stream);
+        b = exl3k::DecodeBatch{};
+        wgs = 0;
+        return from_hip(e);
+    };
+    for (size_t i = 0; i < count; ++i) {
+        const exl3_decode_desc &d = descs[i];
+        const size_t units = (d.k / 16) * ((d.n + 127) / 128);
+        const size_t mwgs = (units + exl3k::kDecodeWaves - 1) / exl3k::kDecodeWaves;
+        // a grid holds fewer than 2^32 threads
+        if (b.count == exl3k::kDecodeBatchMax || wgs + mwgs > (size_t)0xffffff) {
+            const exl3_status st = flush();
+            if (st != EXL3_OK) return st;
         }
-        const exl3_status st = flush();
-        if (st != EXL3_OK) return st;
+        b.src[b.count] = d.src;
+        b.out[b.count] = d.out;
+        b.k[b.count] = d.k;
+        b.n[b.count] = d.n;
+        b.bits[b.count] = (int)d.bits;
+        b.wg_begin[b.count] = (unsigned)wgs;
+        ++b.count;
+        wgs += mwgs;
     }
-    return EXL3_OK;
+    return flush();
 }
 
 exl3_status exl3_hip_decode(const void *src, exl3_layout layout, unsigned bits, unsigned codebook, size_t k, size_t n,

@@ -68,135 +68,101 @@ hipError_t launch_zero(void *ptr, size_t bytes, hipStream_t stream) {
 }
 
 // ============================================================== decode
-// One workgroup block: one 16-row tile row rk, 16 consecutive tile columns
-// starting at tile bx * 16 of the slice.  Lane (wave w, lane l): tile w*4 + l/16,
-// run c = l%8, h = (l%16)/8.
-constexpr int kDecodePitch = 16 * 16 + 8;
+// A unit is one tile row of 8 tiles (16 rows x 128 columns) and belongs to one wave:
+// lane 8 t + j decodes chunk j of tile t (decode_chunk: columns j and j + 8 of it, all
+// 16 rows, two rows per word).  Neighbouring lanes trade halves (one DPP move and one
+// v_perm per word), so that a word is two neighbouring columns of one row, and the wave
+// turns the unit in its own LDS rows (272 bytes apart: 4-byte writes and 16-byte reads
+// without bank conflicts; no barrier, a wave's LDS accesses stay in order) into
+// 256-byte row segments.
+// Bound: HBM.  The projections of a layer of hidden 2048 (k / v 512, 6144 wide MLP, 6 / 4
+// / 3 bits, 121 MB) in one batch 32.5 -> 23.1 us, 5.3 TB/s where a large copy reaches
+// 5.1; against a launch per rate, runs of 16 positions loaded word by word and turned
+// through 2-byte LDS writes.  A second unit per wave, its words loaded ahead, 23.9 us;
+// four 29.1 (fewer waves in flight).
+constexpr int kDecodeRowWords = 68;
 template <int K, int CB>
-__device__ __forceinline__ void decode_block(const uint8_t *__restrict__ src, int records_layout, size_t k, size_t n,
-                                             size_t first_tile, size_t tile_count, uint16_t *__restrict__ out,
-                                             size_t bx, size_t rk, uint16_t *tb) {
-    constexpr int PITCH = kDecodePitch;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const size_t t0 = bx * 16;  // first tile (relative to first_tile) of this workgroup
-    const int tl = wave * 4 + (lane >> 4);
-    const int c = lane & 7, h = (lane >> 3) & 1;
-    if (t0 + tl < tile_count) {
-        const uint32_t *tile = tile_ptr<K>(src, records_layout, k, n, rk, first_tile + t0 + tl);
-        uint32_t w[RunGeo<K>::NW];
-        load_run_words<K>(tile, c, h, w);
-        u4 a1, a2;
-        decode_run<K, CB>(w, a1, a2);
-        const uint32_t p1[4] = {a1.x, a1.y, a1.z, a1.w}, p2[4] = {a2.x, a2.y, a2.z, a2.w};
+__device__ __forceinline__ void decode_unit(const uint8_t *__restrict__ src, int records_layout, size_t k, size_t n,
+                                            size_t rk, size_t block, size_t first_tile, size_t tile_count,
+                                            uint16_t *__restrict__ out, uint32_t *rows) {
+    const int lane = threadIdx.x & 63, j = lane & 7, odd = j & 1;
+    const size_t t0 = block * 8 + (lane >> 3), t = t0 < tile_count ? t0 : tile_count - 1;  // past the end: not stored
+    uint32_t w[K];
+    load_chunk<K>((const uint8_t *)(tile_ptr<K>(src, records_layout, k, n, rk, first_tile + t) + j * K), w);
+    const uint32_t p1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)w[K - 1], 0x121, 0xF, 0xF, false);  // row_ror:1
+    const uint32_t p9 = (uint32_t)__builtin_amdgcn_mov_dpp((int)w[K - 1], 0x129, 0xF, 0xF, false);  // row_ror:9
+    uint32_t first = j == 0 ? ~0u : 0u;
+    asm("" : "+v"(first));  // a mask: v_bfi_b32, not a select on vcc
+    u4 fr[4];
+    decode_chunk<K, CB>(w, (first & p9) | (~first & p1), fr);
+    // words of an even lane: rows 2 v of columns j, j + 1; of an odd one: rows 2 v + 1 of j - 1, j
+    const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
+    uint32_t *dst = rows + odd * kDecodeRowWords + (lane >> 3) * 8 + (j >> 1);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        const uint32_t p[4] = {fr[f].x, fr[f].y, fr[f].z, fr[f].w};
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int r0 = run_slot_row(h, 2 * v), r1 = run_slot_row(h, 2 * v + 1);
-            tb[r0 * PITCH + tl * 16 + c] = (uint16_t)(p1[v] & 0xffffu);
-            tb[r1 * PITCH + tl * 16 + c] = (uint16_t)(p1[v] >> 16);
-            tb[r0 * PITCH + tl * 16 + c + 8] = (uint16_t)(p2[v] & 0xffffu);
-            tb[r1 * PITCH + tl * 16 + c + 8] = (uint16_t)(p2[v] >> 16);
+            const uint32_t q = (uint32_t)__builtin_amdgcn_mov_dpp((int)p[v], 0xB1, 0xF, 0xF, false);  // lane ^ 1
+            dst[(8 * (f & 1) + 2 * v) * kDecodeRowWords + 4 * (f >> 1)] = __builtin_amdgcn_perm(q, p[v], sel);
         }
     }
-    __syncthreads();
-    const size_t count = tile_count * 16;  // output row length
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const size_t width = tile_count * 16, c0 = block * 128 + (lane & 15) * 8;  // output row length, column
+    if (c0 < width) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int ch = tid + 256 * i;      // 16 rows x 32 chunks of 8 halves
-        const int row = ch >> 5, col8 = ch & 31;
-        const int tl2 = col8 >> 1;
-        if (t0 + tl2 < tile_count) {
-            const u4 v = *(const u4 *)(tb + row * PITCH + col8 * 8);
+        for (int i = 0; i < 4; ++i) {
+            const int row = 4 * i + (lane >> 4);
+            const u4 v = *(const u4 *)(rows + row * kDecodeRowWords + (lane & 15) * 4);
             // streaming store: the fp16 output is written once and not read back here
-            __builtin_nontemporal_store(v, (u4 *)(out + (rk * 16 + row) * count + (t0 + tl2) * 16 + (col8 & 1) * 8));
+            __builtin_nontemporal_store(v, (u4 *)(out + (rk * 16 + row) * width + c0));
         }
     }
 }
 
+// columns [16 first_tile, + 16 tile_count) of one matrix; grid (column blocks, tile rows)
 template <int K, int CB>
-__global__ __launch_bounds__(256) void decode_kernel(const uint8_t *__restrict__ src, int records_layout, size_t k,
-                                                     size_t n, size_t first_tile, size_t tile_count,
-                                                     uint16_t *__restrict__ out) {
-    __shared__ uint16_t tb[16 * kDecodePitch];
-    decode_block<K, CB>(src, records_layout, k, n, first_tile, tile_count, out, blockIdx.x, blockIdx.y, tb);
+__global__ __launch_bounds__(kDecodeWaves * 64) void decode_kernel(const uint8_t *__restrict__ src,
+                                                                   int records_layout, size_t k, size_t n,
+                                                                   size_t first_tile, size_t tile_count,
+                                                                   uint16_t *__restrict__ out) {
+    __shared__ __attribute__((aligned(16))) uint32_t turn[kDecodeWaves][16 * kDecodeRowWords];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const size_t block = (size_t)blockIdx.x * kDecodeWaves + wave;
+    if (block * 8 < tile_count)  // whole waves, no barrier follows
+        decode_unit<K, CB>(src, records_layout, k, n, blockIdx.y, block, first_tile, tile_count, out, turn[wave]);
 }
 
-// Several whole matrices of one rate in one launch: workgroup w belongs to the
-// matrix m whose range [wg_begin[m], wg_begin[m + 1]) holds it, and decodes its
-// kDecodeBlocksPerWg consecutive blocks b (bx, rk) = (b % gx, b / gx), gx =
-// ceil(n / 256), from b = kDecodeBlocksPerWg (w - wg_begin[m]): a tile row's
-// neighbouring 256-column blocks.  The next block's stream words are loaded
-// while the current one is decoded, transposed (two LDS buffers) and stored, so
-// a workgroup keeps a block's loads in flight behind its stores.
-template <int K>
-__device__ __forceinline__ bool decode_block_load(const uint8_t *__restrict__ src, int records_layout, size_t k,
-                                                  size_t n, size_t tile_count, size_t gx, size_t b,
-                                                  uint32_t (&w)[RunGeo<K>::NW]) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const size_t bx = b % gx, rk = b / gx, t0 = bx * 16;
-    const int tl = wave * 4 + (lane >> 4);
-    const int c = lane & 7, h = (lane >> 3) & 1;
-    if (t0 + tl >= tile_count) return false;
-    load_run_words<K>(tile_ptr<K>(src, records_layout, k, n, rk, t0 + tl), c, h, w);
-    return true;
+// Several whole matrices, of any rates, in one launch.  Workgroup w belongs to the matrix
+// m whose range [wg_begin[m], wg_begin[m + 1]) holds it; its waves take neighbouring units.
+template <int K, int CB>
+__device__ __forceinline__ void decode_unit_of(const DecodeBatch &batch, int m, int records_layout, uint32_t *rows) {
+    const size_t k = batch.k[m], n = batch.n[m];
+    const unsigned gx = (unsigned)((n + 127) >> 7);
+    const unsigned u = (blockIdx.x - batch.wg_begin[m]) * kDecodeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned rk = u / gx;
+    if (rk < (unsigned)(k >> 4))  // whole waves, no barrier follows
+        decode_unit<K, CB>((const uint8_t *)batch.src[m], records_layout, k, n, rk, u - rk * gx, 0, n >> 4,
+                           batch.out[m], rows);
 }
 
-template <int K, int CB>
-__device__ __forceinline__ void decode_block_store(const uint32_t (&w)[RunGeo<K>::NW], bool valid, size_t tile_count,
-                                                   size_t gx, size_t b, uint16_t *__restrict__ out, uint16_t *tb) {
-    constexpr int PITCH = kDecodePitch;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const size_t bx = b % gx, rk = b / gx, t0 = bx * 16;
-    const int tl = wave * 4 + (lane >> 4);
-    const int c = lane & 7, h = (lane >> 3) & 1;
-    if (valid) {
-        u4 a1, a2;
-        decode_run<K, CB>(w, a1, a2);
-        const uint32_t p1[4] = {a1.x, a1.y, a1.z, a1.w}, p2[4] = {a2.x, a2.y, a2.z, a2.w};
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int r0 = run_slot_row(h, 2 * v), r1 = run_slot_row(h, 2 * v + 1);
-            tb[r0 * PITCH + tl * 16 + c] = (uint16_t)(p1[v] & 0xffffu);
-            tb[r1 * PITCH + tl * 16 + c] = (uint16_t)(p1[v] >> 16);
-            tb[r0 * PITCH + tl * 16 + c + 8] = (uint16_t)(p2[v] & 0xffffu);
-            tb[r1 * PITCH + tl * 16 + c + 8] = (uint16_t)(p2[v] >> 16);
-        }
-    }
-    __syncthreads();
-    const size_t count = tile_count * 16;  // output row length
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int ch = tid + 256 * i;  // 16 rows x 32 chunks of 8 halves
-        const int row = ch >> 5, col8 = ch & 31;
-        const int tl2 = col8 >> 1;
-        if (t0 + tl2 < tile_count) {
-            const u4 v = *(const u4 *)(tb + row * PITCH + col8 * 8);
-            __builtin_nontemporal_store(v, (u4 *)(out + (rk * 16 + row) * count + (t0 + tl2) * 16 + (col8 & 1) * 8));
-        }
-    }
-}
-
-template <int K, int CB>
-__global__ __launch_bounds__(256) void decode_batch_kernel(DecodeBatch batch, int records_layout) {
-    __shared__ uint16_t tb[2][16 * kDecodePitch];  // one block's transpose while the other's is read
+template <int CB>
+__global__ __launch_bounds__(kDecodeWaves * 64) void decode_batch_kernel(DecodeBatch batch, int records_layout) {
+    __shared__ __attribute__((aligned(16))) uint32_t turn[kDecodeWaves][16 * kDecodeRowWords];
     const unsigned w = blockIdx.x;
     int m = 0;
     for (int i = 1; i < batch.count; ++i)
         if (w >= batch.wg_begin[i]) m = i;
-    const size_t k = batch.k[m], n = batch.n[m];
-    const size_t tiles = n / 16, gx = (tiles + 15) / 16, nblk = (k / 16) * gx;
-    const size_t b0 = (size_t)(w - batch.wg_begin[m]) * kDecodeBlocksPerWg;
-    const uint8_t *src = (const uint8_t *)batch.src[m];
-    uint32_t wa[RunGeo<K>::NW], wb[RunGeo<K>::NW];
-    bool va = decode_block_load<K>(src, records_layout, k, n, tiles, gx, b0, wa), vb = false;
-#pragma unroll
-    for (int j = 0; j < kDecodeBlocksPerWg; j += 2) {  // two register sets: no copy of words in flight
-        if (b0 + j >= nblk) break;  // uniform
-        if (b0 + j + 1 < nblk) vb = decode_block_load<K>(src, records_layout, k, n, tiles, gx, b0 + j + 1, wb);
-        decode_block_store<K, CB>(wa, va, tiles, gx, b0 + j, batch.out[m], tb[0]);
-        if (b0 + j + 1 >= nblk) break;
-        if (j + 2 < kDecodeBlocksPerWg && b0 + j + 2 < nblk)
-            va = decode_block_load<K>(src, records_layout, k, n, tiles, gx, b0 + j + 2, wa);
-        decode_block_store<K, CB>(wb, vb, tiles, gx, b0 + j + 1, batch.out[m], tb[1]);
+    uint32_t *rows = turn[threadIdx.x >> 6];
+    switch (batch.bits[m]) {
+    case 1: decode_unit_of<1, CB>(batch, m, records_layout, rows); break;
+    case 2: decode_unit_of<2, CB>(batch, m, records_layout, rows); break;
+    case 3: decode_unit_of<3, CB>(batch, m, records_layout, rows); break;
+    case 4: decode_unit_of<4, CB>(batch, m, records_layout, rows); break;
+    case 5: decode_unit_of<5, CB>(batch, m, records_layout, rows); break;
+    case 6: decode_unit_of<6, CB>(batch, m, records_layout, rows); break;
+    case 7: decode_unit_of<7, CB>(batch, m, records_layout, rows); break;
+    default: decode_unit_of<8, CB>(batch, m, records_layout, rows); break;
     }
 }
 
@@ -204,7 +170,8 @@ template <int K>
 static hipError_t launch_decode_k(const void *src, int rl, int cb, size_t k, size_t n, size_t first, size_t count,
                                   uint16_t *out, hipStream_t stream) {
     const size_t tiles = count / 16;
-    const dim3 grid((unsigned)((tiles + 15) / 16), (unsigned)(k / 16)), block(256);
+    const dim3 grid((unsigned)((tiles + 8 * kDecodeWaves - 1) / (8 * kDecodeWaves)), (unsigned)(k / 16));
+    const dim3 block(kDecodeWaves * 64);
     const uint8_t *s = (const uint8_t *)src;
     switch (cb) {
     case 0: decode_kernel<K, 0><<<grid, block, 0, stream>>>(s, rl, k, n, first / 16, tiles, out); break;
@@ -214,27 +181,14 @@ static hipError_t launch_decode_k(const void *src, int rl, int cb, size_t k, siz
     return hipGetLastError();
 }
 
-template <int K>
-static hipError_t launch_decode_batch_k(const DecodeBatch &b, int rl, int cb, unsigned wgs, hipStream_t stream) {
+hipError_t launch_decode_batch(const DecodeBatch &b, int rl, int cb, unsigned wgs, hipStream_t stream) {
+    const dim3 grid(wgs), block(kDecodeWaves * 64);
     switch (cb) {
-    case 0: decode_batch_kernel<K, 0><<<dim3(wgs), dim3(256), 0, stream>>>(b, rl); break;
-    case 1: decode_batch_kernel<K, 1><<<dim3(wgs), dim3(256), 0, stream>>>(b, rl); break;
-    default: decode_batch_kernel<K, 2><<<dim3(wgs), dim3(256), 0, stream>>>(b, rl); break;
+    case 0: decode_batch_kernel<0><<<grid, block, 0, stream>>>(b, rl); break;
+    case 1: decode_batch_kernel<1><<<grid, block, 0, stream>>>(b, rl); break;
+    default: decode_batch_kernel<2><<<grid, block, 0, stream>>>(b, rl); break;
     }
     return hipGetLastError();
-}
-
-hipError_t launch_decode_batch(const DecodeBatch &b, int rl, int bits, int cb, unsigned wgs, hipStream_t stream) {
-    switch (bits) {
-    case 1: return launch_decode_batch_k<1>(b, rl, cb, wgs, stream);
-    case 2: return launch_decode_batch_k<2>(b, rl, cb, wgs, stream);
-    case 3: return launch_decode_batch_k<3>(b, rl, cb, wgs, stream);
-    case 4: return launch_decode_batch_k<4>(b, rl, cb, wgs, stream);
-    case 5: return launch_decode_batch_k<5>(b, rl, cb, wgs, stream);
-    case 6: return launch_decode_batch_k<6>(b, rl, cb, wgs, stream);
-    case 7: return launch_decode_batch_k<7>(b, rl, cb, wgs, stream);
-    default: return launch_decode_batch_k<8>(b, rl, cb, wgs, stream);
-    }
 }
 
 hipError_t launch_decode(const void *src, int rl, int bits, int cb, size_t k, size_t n, size_t first, size_t count,

@@ -70,15 +70,15 @@ struct GemvTargets {
     int count;
 };
 
-// Whole matrices of one rate decoded by one launch (decode_batch_kernel).
+// Whole matrices decoded by one launch (decode_batch_kernel).
 constexpr int kDecodeBatchMax = 32;
-// 256-column decode blocks per workgroup of a batch launch (even)
-constexpr unsigned kDecodeBlocksPerWg = 2;
+constexpr int kDecodeWaves = 4;  // waves of a workgroup, one unit of 16 rows x 128 columns each
 struct DecodeBatch {
     const void *src[kDecodeBatchMax];
     uint16_t *out[kDecodeBatchMax];
     size_t k[kDecodeBatchMax], n[kDecodeBatchMax];
-    unsigned wg_begin[kDecodeBatchMax];  // first workgroup of each matrix: ceil((k/16) ceil(n/256) / kDecodeBlocksPerWg) each
+    unsigned wg_begin[kDecodeBatchMax];  // first workgroup of each matrix: ceil((k/16) ceil(n/128) / kDecodeWaves) each
+    int bits[kDecodeBatchMax];
     int count;
 };
 
@@ -135,7 +135,7 @@ hipError_t launch_gemm_targets(const GemvTargets &targets, int bits, int cb, con
                                size_t x_stride, int y_f16, void *workspace, const GemmPlan &plan, hipStream_t stream);
 hipError_t launch_decode(const void *src, int records_layout, int bits, int cb, size_t k, size_t n,
                          size_t first, size_t count, uint16_t *out, hipStream_t stream);
-hipError_t launch_decode_batch(const DecodeBatch &batch, int records_layout, int bits, int cb, unsigned workgroups,
+hipError_t launch_decode_batch(const DecodeBatch &batch, int records_layout, int cb, unsigned workgroups,
                                hipStream_t stream);
 hipError_t launch_reconstruct(const void *src, int records_layout, const uint16_t *su, const uint16_t *sv,
                               int bits, int cb, size_t k, size_t n, size_t first, size_t count, uint16_t *out,
