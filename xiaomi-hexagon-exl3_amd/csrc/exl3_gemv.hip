@@ -202,13 +202,14 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
                            : dummy + lane_off;
     };
     uint32_t buf[D][K];
-    // Ring slots issued before the prep barrier.  Two in the prep of more than one block per
-    // wave (against one: 4 layers of hidden 4096 at 4 rows 245.9 -> 240.4 us, of hidden 2048
-    // at 16 rows 195.3 -> 190.8; four lose 3 to 8 %).  In the short one-block prep two from 5
-    // bits on (k = 4096, n = 14336 at 6 bits 16.10 -> 15.28 us), none below, where they delay
-    // the activations of the other workgroups (k = 14336, n = 4096 at 4 bits 12.67 -> 12.86).
-    constexpr int EARLY = 2;
-    constexpr bool kEarlyOne = K >= 5;
+    // Ring slots issued before the prep barrier, behind the activation loads: two from 5 bits
+    // on and at 9..16 rows (k = 4096, n = 14336 at 6 bits 16.8 -> 16.1 us; 4 layers of hidden
+    // 2048 at 16 rows 194.8 -> 189.7), else one, and none in the one-block prep of the lower
+    // rates, where they delay the activations of the other workgroups (4 layers of hidden
+    // 2048 at 1 row 115.9 -> 118.4 us with two everywhere, at 4 bits k = 14336, n = 4096 12.6
+    // -> 12.8; hidden 4096 at 4 rows gains 230 -> 226).  Four lose 3 to 8 %.
+    constexpr int EARLY = K >= 5 || MODE == 1 ? 2 : 1;
+    constexpr bool kEarlyOne = EARLY == 2;
 
     // 1-2. prep: xh = H128(x[r] su) per (kb, row) block of the workgroup, as
     // fp16 hi = rn(xh) and lo = rn(xh - hi) into the B fragments.  Unit q of
@@ -397,7 +398,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
     __syncthreads();
     stamps.mark(1);
     if constexpr (MODE == 1) __builtin_amdgcn_s_setprio(0);
-    if (MODE == 2 || (!kEarlyOne && nblk <= W)) {  // not issued by the prep
+    if constexpr (EARLY == 1) {
+        if (MODE == 2 || nblk <= W) load_chunk<K>(group_src(0), buf[0]);
+    } else if constexpr (MODE == 2) {
 #pragma unroll
         for (int d = 0; d < EARLY; ++d) load_chunk<K>(group_src(d), buf[d]);
     }
@@ -699,14 +702,24 @@ GemvPlan gemv_plan(size_t k, size_t n, size_t rows) {
     s = (p.kbs + (p.kbs + s - 1) / s - 1) / ((p.kbs + s - 1) / s);
     // a workgroup's B fragments must fit its LDS budget and a wave prepares at
     // most kGemvPrepMax (kb, row) blocks; one kb per workgroup always fits
-    for (;;) {
-        const size_t nkb = ((size_t)p.kbs + s - 1) / s;
+    auto serves = [&](int splits) {
+        const size_t nkb = ((size_t)p.kbs + splits - 1) / splits;
         const bool ok_lds = nkb * gemv_frag_bytes_per_kb(rows) <= (rows > 8 ? kGemvFragLds16 : kGemvFragLds);
         // above 16 rows the activations are prepared once per call (gemv_xprep_kernel)
         const bool ok_prep = rows > 16 || (nkb * rows + kGemvWaves - 1) / kGemvWaves <= (size_t)kGemvPrepMax;
-        if ((ok_lds && ok_prep) || s >= p.kbs) break;
-        ++s;
-    }
+        return ok_lds && ok_prep;
+    };
+    // between one and two workgroups per CU some CUs run two in turn and others idle: one
+    // per CU is better where that leaves the busiest CU fewer records (q/k/v 4096 + 2 x 1024
+    // of k = 4096, 8 -> 5 splits: rows 1 10.6 -> 9.4 us, rows 8 12.3 -> 10.7; k = 8192,
+    // n = 3072, 16 -> 10: 9.2 -> 8.9 and 11.3 -> 10.9).  With as many records either way
+    // neither is better throughout (k = 14336, n = 4096 16 splits 13.1, 8 splits 14.4;
+    // 2 x 14336 of k = 4096 2 splits 23.5, none 22.1)
+    const int one = 256 / p.nbs, rounds = (p.nbs * s + 255) / 256;
+    if (rows <= (size_t)kGemvSingleMaxRows && rounds > 1 && one >= 1 && serves(one) &&
+        (p.kbs + one - 1) / one < rounds * ((p.kbs + s - 1) / s))
+        s = one;
+    while (!serves(s) && s < p.kbs) ++s;
     p.splits = s;
     p.nkw = (p.kbs + s - 1) / s;
     p.partials_off = 0;  // the exchange
