@@ -109,8 +109,19 @@ exl3_status call_workspace(size_t need, F want, hipStream_t stream, void **works
 // (rows 15..32: the GEMM for one matrix, the GEMV for a group of them), so that one
 // workspace serves all smaller calls of the same (k, n) in turn (every plan starts
 // with the same exchange region).
+// The last sizes asked for are kept per thread (a pure function of its arguments): a call
+// of 37 rows otherwise plans the smaller row counts again each time (1.7 us of host time).
 size_t mul_mat_need(size_t k, size_t n, size_t rows, bool tails) {
     if (!valid_matrix(k, n, 128) || rows < 1 || rows > kMaxRows) return 0;
+    struct Kept {
+        size_t k, n, rows, need;
+        bool tails;
+    };
+    constexpr size_t kKept = 16;
+    thread_local Kept kept[kKept] = {};
+    thread_local size_t next = 0;
+    for (const Kept &e : kept)
+        if (e.k == k && e.n == n && e.rows == rows && e.tails == tails) return e.need;
     size_t need = 0;
     const size_t gemv_rows = rows < (size_t)exl3k::kGemvMaxRows ? rows : (size_t)exl3k::kGemvMaxRows;
     for (size_t r = 1; r <= gemv_rows; ++r) {
@@ -118,6 +129,8 @@ size_t mul_mat_need(size_t k, size_t n, size_t rows, bool tails) {
         need = std::max(need, p.fits ? p.bytes : exl3k::gemm_plan(k, n, r, tails).bytes);
     }
     for_gemm_plans(rows, [&](size_t r) { need = std::max(need, exl3k::gemm_plan(k, n, r, tails).bytes); });
+    kept[next] = Kept{k, n, rows, need, tails};
+    next = (next + 1) % kKept;
     return need;
 }
 

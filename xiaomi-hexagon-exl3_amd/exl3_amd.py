@@ -171,10 +171,11 @@ def lib():
     return _LIB
 
 
+# Pointers and streams go to ctypes as plain integers (argtypes are c_void_p): no object per
+# argument (an eager one-row call of 2048 x 6144 is bound by its host time: 9.4 -> 8.4 us a call).
 def _stream(stream=None):
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return (stream if stream is not None else torch.cuda.current_stream()).cuda_stream
 
 
 def _check(status, what):
@@ -183,7 +184,7 @@ def _check(status, what):
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def workspace_bytes(k, n, rows):
