@@ -591,7 +591,7 @@ template <int K>
 static hipError_t launch_get_rows_k(const void *records, int cb, size_t k, size_t n, const int32_t *ids,
                                     size_t ids_stride, size_t count, void *out, int out_f16, size_t out_stride,
                                     int *bad_ids, hipStream_t stream) {
-    const size_t gy = count < 32768 ? count : 32768;
+    const size_t gy = count < 65535 ? count : 65535;  // z then stays within 65,535 for any count
     const dim3 grid((unsigned)(k / 128), (unsigned)gy, (unsigned)((count + gy - 1) / gy)), block(kGetRowsThreads);
     const uint8_t *rec = (const uint8_t *)records;
     switch (cb) {
