@@ -234,11 +234,13 @@ typedef struct exl3_matrix_desc {
 /* y_i = layer_i(x) for 1..4 matrices that share k, bits, codebook, x and rows
  * (the q/k/v or gate/up projections of one decoder layer): at rows <=
  * exl3_hip_gemv_max_rows() one GEMV launch serves all of them, so the launch and
- * its latency chain are paid once; larger row counts run one GEMM for all of them,
- * or, where the workspace only holds that, one exl3_hip_mul_mat per matrix.  Each y_i is the exl3_hip_mul_mat result within the layer
- * tolerance (the split of k follows the total width, so the summation order may
- * differ from a single call's).  workspace: >= exl3_hip_mul_mat_workspace_bytes(k,
- * sum of n_i, rows), or NULL for the internal one.  This entry point has no
+ * its latency chain are paid once; larger row counts run one GEMM launch for all of
+ * them, or, where the workspace only holds that, one exl3_hip_mul_mat per matrix (the
+ * same bits).  Each y_i is the exl3_hip_mul_mat result within the layer tolerance (in
+ * the GEMV the split of k follows the total width, so the summation order may differ
+ * from a single call's).  workspace: >= exl3_hip_mul_mat_workspace_bytes(k, n, rows) of
+ * every n_i and of their sum; exl3_hip_mul_mat_group_workspace_bytes also holds the one
+ * GEMM launch; NULL for the internal one.  This entry point has no
  * counterpart in the reference, whose ggml op multiplies one matrix per call. */
 exl3_status exl3_hip_mul_mat_group(const exl3_matrix_desc *mats, size_t count, unsigned bits, unsigned codebook,
                                    size_t k, const void *x, exl3_dtype xt, size_t rows, size_t x_row_stride,
@@ -247,8 +249,8 @@ exl3_status exl3_hip_mul_mat_group(const exl3_matrix_desc *mats, size_t count, u
 /* Workspace bytes of an exl3_hip_mul_mat_group call: the most any row count
  * 1..rows needs to run as one GEMV or one GEMM over all matrices (each has its own
  * prepared activations and split partials there).  0 for invalid arguments.  Calls
- * also take less: as much as the GEMV over the total width and each
- * exl3_hip_mul_mat need, without the space that only faster plans use. */
+ * also take less: as much as exl3_hip_mul_mat needs for the total width and for each
+ * matrix. */
 size_t exl3_hip_mul_mat_group_workspace_bytes(size_t k, const size_t *n, size_t count, size_t rows);
 
 /* The ggml op on ggml views, replacing ggml_exl3_mul_mat (src/exl3-ggml.cpp:51-92)

@@ -64,6 +64,24 @@ def test_noalloc_matches_mul_mat_on_consecutive_calls(amd):
             print(f"  noalloc call {i}: k={k} n={n} bits={bits} rows={rows} {out_dtype}: equal", flush=True)
 
 
+def test_noalloc_matches_mul_mat_beyond_one_tile_per_cu(amd):
+    """384 tiles of 512 rows (k = 2048, n = 6144, 4096 rows; 32 MiB of workspace): with the 64 MiB
+    array, a workspace of the documented size and a larger one, the same bits."""
+    import torch
+    k, n, bits, rows = 2048, 6144, 2, 4096
+    rec = make_layer(2300, k, n, bits)
+    g = torch.Generator(device="cuda").manual_seed(2301)
+    x = torch.randn((rows, k), generator=g, device="cuda").half()
+    print(f"  noalloc k={k} n={n} rows={rows}", flush=True)
+    need = amd.workspace_bytes(k, n, rows)
+    assert need <= 64 << 20
+    y = torch.full((rows, n), float("nan"), device="cuda")
+    assert noalloc(amd, rec, bits, k, n, x, y) == amd.OK
+    for nbytes in (need, 4 * need):
+        ref = amd.mul_mat(rec, bits, k, n, x, workspace=amd.new_workspace(k, n, rows, nbytes=nbytes))
+        assert torch.equal(y, ref), f"workspace of {nbytes} bytes"
+
+
 def test_noalloc_under_graph_capture(amd):
     """A captured call allocates nothing (global capture mode would fail on an
     allocation); replays with eager work in between equal the eager result."""

@@ -97,12 +97,16 @@ exl3_status internal_workspace(size_t need, size_t want, hipStream_t stream, voi
 }
 
 // A call's workspace: the caller's, of at least `need` bytes, or the internal one, of
-// want() bytes where it may grow.
+// want() bytes where it may grow (a group's one GEMM launch takes more than its calls
+// one by one; the bits are the same either way).
 template <typename F>
 exl3_status call_workspace(size_t need, F want, hipStream_t stream, void **workspace, size_t *bytes) {
     if (!*workspace) return internal_workspace(need, want(), stream, workspace, bytes);
     if (!aligned(*workspace, 256)) return EXL3_INVAL_PARAMS;
     return *bytes < need ? EXL3_WORKSPACE_TOO_SMALL : EXL3_OK;
+}
+exl3_status call_workspace(size_t need, hipStream_t stream, void **workspace, size_t *bytes) {
+    return call_workspace(need, [=] { return need; }, stream, workspace, bytes);
 }
 
 // Largest plan over every row count 1..rows and both paths a row count can take
@@ -111,42 +115,41 @@ exl3_status call_workspace(size_t need, F want, hipStream_t stream, void **works
 // with the same exchange region).
 // The last sizes asked for are kept per thread (a pure function of its arguments): a call
 // of 37 rows otherwise plans the smaller row counts again each time (1.7 us of host time).
-size_t mul_mat_need(size_t k, size_t n, size_t rows, bool tails) {
+size_t mul_mat_need(size_t k, size_t n, size_t rows) {
     if (!valid_matrix(k, n, 128) || rows < 1 || rows > kMaxRows) return 0;
     struct Kept {
         size_t k, n, rows, need;
-        bool tails;
     };
     constexpr size_t kKept = 16;
     thread_local Kept kept[kKept] = {};
     thread_local size_t next = 0;
     for (const Kept &e : kept)
-        if (e.k == k && e.n == n && e.rows == rows && e.tails == tails) return e.need;
+        if (e.k == k && e.n == n && e.rows == rows) return e.need;
     size_t need = 0;
     const size_t gemv_rows = rows < (size_t)exl3k::kGemvMaxRows ? rows : (size_t)exl3k::kGemvMaxRows;
     for (size_t r = 1; r <= gemv_rows; ++r) {
         const exl3k::GemvPlan p = exl3k::gemv_plan(k, n, r);
-        need = std::max(need, p.fits ? p.bytes : exl3k::gemm_plan(k, n, r, tails).bytes);
+        need = std::max(need, p.fits ? p.bytes : exl3k::gemm_plan(k, n, r).bytes);
     }
-    for_gemm_plans(rows, [&](size_t r) { need = std::max(need, exl3k::gemm_plan(k, n, r, tails).bytes); });
-    kept[next] = Kept{k, n, rows, need, tails};
+    for_gemm_plans(rows, [&](size_t r) { need = std::max(need, exl3k::gemm_plan(k, n, r).bytes); });
+    kept[next] = Kept{k, n, rows, need};
     next = (next + 1) % kKept;
     return need;
 }
 
 // The same for a grouped call: the least it takes (one GEMV launch over the total
-// width, or one call per matrix), and with `fused` the GEMM launch for all of them.
+// width, or one call per matrix), and with `fused` the one GEMM launch for all of them.
 size_t group_need(size_t k, const size_t *n, size_t count, size_t rows, bool fused) {
     if (!n || count < 1 || count > (size_t)exl3k::kGemvMaxTargets) return 0;
     size_t n_total = 0, need = 0;
     for (size_t i = 0; i < count; ++i) {
-        const size_t b = mul_mat_need(k, n[i], rows, fused);
+        const size_t b = mul_mat_need(k, n[i], rows);
         if (!b) return 0;
         need = std::max(need, b);
         n_total += n[i];
     }
     if (n_total > kMaxDim) return 0;
-    need = std::max(need, mul_mat_need(k, n_total, rows, fused));
+    need = std::max(need, mul_mat_need(k, n_total, rows));
     if (fused && count > 1)
         for_gemm_plans(rows, [&](size_t r) {
             const exl3k::GemmPlan p = exl3k::gemm_plan_group(k, n, (int)count, r);
@@ -268,7 +271,7 @@ int exl3_hip_supports_op(exl3_op op, const exl3_tensor_info *dst, const exl3_ten
     return 0;
 }
 
-size_t exl3_hip_mul_mat_workspace_bytes(size_t k, size_t n, size_t rows) { return mul_mat_need(k, n, rows, true); }
+size_t exl3_hip_mul_mat_workspace_bytes(size_t k, size_t n, size_t rows) { return mul_mat_need(k, n, rows); }
 
 exl3_status exl3_hip_workspace_init(void *workspace, size_t workspace_bytes, hipStream_t stream) {
     if (!workspace) {  // the internal workspace of (current device, stream), if there is one
@@ -319,8 +322,7 @@ static exl3_status mul_mat_impl(const void *records, unsigned bits, unsigned cod
     if (!records || !x || !y || !aligned(records, 16)) return EXL3_INVAL_PARAMS;
     if (!aligned(x, dtype_size(xt)) || !aligned(y, dtype_size(yt))) return EXL3_INVAL_PARAMS;
     if (x_row_stride < k || y_row_stride < n) return EXL3_INVAL_PARAMS;
-    const exl3_status st = call_workspace(mul_mat_need(k, n, rows, false), [&] { return mul_mat_need(k, n, rows, true); },
-                                          stream, &workspace, &workspace_bytes);
+    const exl3_status st = call_workspace(mul_mat_need(k, n, rows), stream, &workspace, &workspace_bytes);
     if (st != EXL3_OK) return st;
     exl3k::GemvTargets tg{};
     tg.records[0] = (const uint8_t *)records;
@@ -334,10 +336,8 @@ static exl3_status mul_mat_impl(const void *records, unsigned bits, unsigned cod
     if (exl3k::gemv_serves_single(k, n, rows))
         return from_hip(exl3k::launch_gemv_targets(tg, (int)bits, (int)codebook, x, xf, rows, x_row_stride, yf,
                                                    workspace, exl3k::gemv_plan(k, n, rows), stream));
-    exl3k::GemmPlan plan = exl3k::gemm_plan(k, n, rows, true);
-    if (plan.bytes > workspace_bytes) plan = exl3k::gemm_plan(k, n, rows, false);
     return from_hip(exl3k::launch_gemm_targets(tg, (int)bits, (int)codebook, x, xf, rows, x_row_stride, yf, workspace,
-                                               plan, stream));
+                                               exl3k::gemm_plan(k, n, rows), stream));
 }
 
 exl3_status exl3_hip_mul_mat(const void *records, unsigned bits, unsigned codebook, size_t k, size_t n, const void *x,
@@ -440,9 +440,7 @@ exl3_status exl3_hip_mul_mat_nd(const void *records, unsigned bits, unsigned cod
     if (!exl3_hip_supports_mul_mat(bits, codebook, k, n, rows, xt, yt) || !records || !x || !y)
         return EXL3_INVAL_PARAMS;
     // every call below needs at most this
-    const exl3_status wst = call_workspace(mul_mat_need(k, n, rows, false),
-                                           [&] { return mul_mat_need(k, n, rows, true); }, stream, &workspace,
-                                           &workspace_bytes);
+    const exl3_status wst = call_workspace(mul_mat_need(k, n, rows), stream, &workspace, &workspace_bytes);
     if (wst != EXL3_OK) return wst;
     // Row dimensions 1, 2, 3 in order join one run while both views step through
     // them with one row stride (a run's stride at least a row, as exl3_hip_mul_mat
@@ -614,13 +612,13 @@ exl3_status exl3_hip_pack_records(const uint16_t *packed, const uint16_t *su, co
 
 // Workspace of exl3_hip_iface_matmul: the mul_mat workspace (its counters first,
 // so one zero-fill covers both), then the packed records.
-static size_t iface_records_offset(size_t k, size_t n, size_t batch, bool tails) {
-    return (mul_mat_need(k, n, batch, tails) + 255) & ~(size_t)255;
+static size_t iface_records_offset(size_t k, size_t n, size_t batch) {
+    return (mul_mat_need(k, n, batch) + 255) & ~(size_t)255;
 }
 
 size_t exl3_hip_iface_matmul_workspace_bytes(unsigned bits, size_t k, size_t n, size_t batch) {
     if (bits < 1 || bits > 8 || !valid_matrix(k, n, 128) || batch < 1 || batch > kMaxRows) return 0;
-    return iface_records_offset(k, n, batch, true) + (n / 128) * (k / 128) * ((size_t)2048 * bits + 512);
+    return iface_records_offset(k, n, batch) + (n / 128) * (k / 128) * ((size_t)2048 * bits + 512);
 }
 
 // exl3_iface_matmul (src/hexagon/exl3_service.c:265-305): the argument checks of
@@ -633,10 +631,8 @@ exl3_status exl3_hip_iface_matmul(unsigned bits, unsigned codebook, size_t k, si
     if (!packed || !suh || !svh || !x || !y) return EXL3_INVAL_PARAMS;
     if (!aligned(packed, 16) || !aligned(suh, 16) || !aligned(svh, 16) || !aligned(x, 4) || !aligned(y, 4))
         return EXL3_INVAL_PARAMS;
-    const size_t want = exl3_hip_iface_matmul_workspace_bytes(bits, k, n, batch);
-    const size_t least = iface_records_offset(k, n, batch, false);
-    const size_t need = least + (want - iface_records_offset(k, n, batch, true));
-    exl3_status st = call_workspace(need, [&] { return want; }, stream, &workspace, &workspace_bytes);
+    exl3_status st = call_workspace(exl3_hip_iface_matmul_workspace_bytes(bits, k, n, batch), stream, &workspace,
+                                    &workspace_bytes);
     if (st != EXL3_OK) return st;
     // the GEMV reads the tiles as they are (2048 x 6144, 5 bits, batch 8: 15.0 -> 10.3 us per
     // call against packing records first); the GEMM, which reads each weight once per row
@@ -644,7 +640,7 @@ exl3_status exl3_hip_iface_matmul(unsigned bits, unsigned codebook, size_t k, si
     if (exl3k::gemv_serves_single(k, n, batch))
         return from_hip(exl3k::launch_gemv_tiles(packed, suh, svh, (int)bits, (int)codebook, x, batch, y, n, workspace,
                                                  exl3k::gemv_plan(k, n, batch), stream));
-    const size_t roff = workspace_bytes < want ? least : iface_records_offset(k, n, batch, true);
+    const size_t roff = iface_records_offset(k, n, batch);
     void *records = (uint8_t *)workspace + roff;
     st = exl3_hip_pack_records(packed, suh, svh, bits, k, n, records, stream);
     if (st != EXL3_OK) return st;
@@ -661,5 +657,3 @@ exl3_status exl3_hip_validate_records(const void *records, size_t nbytes, unsign
 }
 
 }  // extern "C"
-
-size_t exl3k::mul_mat_least_workspace(size_t k, size_t n, size_t rows) { return mul_mat_need(k, n, rows, false); }

@@ -182,12 +182,11 @@ template <bool UNIT>
 __device__ __forceinline__ GemmSegment gemm_segment(const GemmGrid &gg, int id) {
     GemmSegment s = gg.seg[0];
 #pragma unroll
-    for (int i = 1; i < kGemmMaxSegments; ++i) {
+    for (int i = 1; i < kGemvMaxTargets; ++i) {
         const GemmSegment &c = gg.seg[i];
         const bool in = i < gg.count && id >= (UNIT ? c.unit0 : c.begin);
         s.begin = in ? c.begin : s.begin;
         s.nb0 = in ? c.nb0 : s.nb0;
-        s.tile0 = in ? c.tile0 : s.tile0;
         s.tiles = in ? c.tiles : s.tiles;
         s.splits = in ? c.splits : s.splits;
         s.kq = in ? c.kq : s.kq;
@@ -319,7 +318,7 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
     const int item = (id & 7) * per_xcd + (id >> 3);
     if (item >= items) return;  // padding, whole workgroups
     const int splits = sg.splits, s = splits > 1 ? item / sg.tiles : 0, ts = item - s * sg.tiles;
-    const int nbt = (sg.tile0 + ts) / gg.mtiles, mt = sg.tile0 + ts - nbt * gg.mtiles;
+    const int nbt = ts / gg.mtiles, mt = ts - nbt * gg.mtiles;
     const int kbs = gg.kbs;
     const GemmColumn col = gemm_column<false>(tg, sg.nb0 + nbt, (size_t)kbs * GB);
     // split s owns kq + (s < kr) records from kb0 (kq = kbs / splits, kr = kbs % splits, from the host)
@@ -534,7 +533,7 @@ __global__ __launch_bounds__(W * 64) void gemm_kernel(
 // of a batch in flight together; the sums go through LDS as [row][column], and wave w then
 // finishes rows 4 w .. 4 w + 3 (h128_wave over the 128 columns, sv, the optional
 // residual), lane l writing columns l and l + 64.
-// ONE: a single target and a single split segment, gg.seg[0] (the other arguments stay
+// ONE: a single target, gg.seg[0] (the other arguments stay
 // unread: with the general form -0.2 to -0.5 us per call at M = 512 and rows 37).
 template <int RB, int W, int SB, bool ONE>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemvTargets tg, GemmGrid gg, int bits,
@@ -547,7 +546,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemvTargets tg, GemmGr
     const GemmSegment sg = ONE ? gg.seg[0] : gemm_segment<true>(gg, (int)blockIdx.x);
     const int splits = sg.splits, u = (int)blockIdx.x - sg.unit0;
     const int vp = u & 1, blk = (u >> 1) % (W * RB), ts = (u >> 1) / (W * RB);
-    const int nbt = (sg.tile0 + ts) / gg.mtiles, mt = sg.tile0 + ts - nbt * gg.mtiles;
+    const int nbt = ts / gg.mtiles, mt = ts - nbt * gg.mtiles;
     const GemmColumn col = gemm_column<ONE>(tg, sg.nb0 + nbt, (size_t)gg.kbs * group_bytes(bits));
     const int nb = col.nb;
     void *y = col.y;
@@ -639,8 +638,8 @@ int gemm_tile_rows(size_t rows) {
     return rows <= 32 ? 32 : rows <= 64 ? 64 : rows <= 128 ? 128 : rows <= 256 ? 256 : 512;
 }
 
-// k splits of a set of `tiles` tiles that run together (summed by gemm_reduce_kernel),
-// at most one split per record.
+// k splits of a matrix of `tiles` tiles (summed by gemm_reduce_kernel), at most one split
+// per record.
 // 32- and 64-row tiles fill the CUs once (one workgroup each); 32-row tiles (4
 // waves, 64 KB of LDS) run two per CU when each split keeps >= 4 records (rows
 // 17..32 at k = 14336, n = 4096: 22.7 -> 21.2 us; at k <= 6144 two per CU with
@@ -677,63 +676,34 @@ static int gemm_splits(int kbs, int tiles, int bm) {
     return s < 1 ? 1 : (s > kbs ? kbs : s);
 }
 
-// Appends the segments of `tiles` tiles over column groups nb0 .. nb0 + nbs - 1: one
-// without a split, or one with, or (tails, 256- and 512-row tiles, more tiles than CUs)
-// the full rounds of one tile per CU without and the last, partial round's tiles with a
-// split that fills the CUs again, where gemm_splits finds one cheaper than a whole round.
-static void gemm_add(GemmPlan &p, GemmSegment *direct, int &nd, GemmSegment *split, int &ns, int nb0, int nbs,
-                     bool tails) {
-    const int tiles = nbs * p.mtiles;
-    int full = 0, s = gemm_splits(p.kbs, tiles, p.bm);
-    if (s == 1) full = tiles;
-    if (tails && p.bm >= 256 && tiles > kGemmTargetWgs && tiles % kGemmTargetWgs) {
-        const int t = gemm_splits(p.kbs, tiles % kGemmTargetWgs, p.bm);
-        if (t > 1) s = t, full = tiles - tiles % kGemmTargetWgs;
-    }
-    GemmSegment g{};
-    g.nb0 = nb0;
-    if (full) {
-        g.tile0 = 0;
-        g.tiles = full;
-        g.splits = 1;
-        g.kq = p.kbs;
-        direct[nd++] = g;
-    }
-    if (full < tiles) {
-        g.tile0 = full;
-        g.tiles = tiles - full;
-        g.splits = s;
-        g.kq = p.kbs / s;
-        g.kr = p.kbs % s;
-        split[ns++] = g;
-    }
-}
-
-static GemmPlan gemm_plan_bm(size_t k, const size_t *n, int count, size_t rows, int bm, bool tails) {
+// The plan is a function of the sizes alone, and a matrix's tiles are split over k all or
+// not at all: a whole tile sums the whole of k in fp32, whatever the other tiles of its
+// round do.  (Splitting only the tiles of a partial last round, 258 to 511 tiles on 256
+// CUs, saves up to 13 % of a call, but puts their sums through the fp16 partials and needs
+// more workspace than the row counts below.)
+static GemmPlan gemm_plan_bm(size_t k, const size_t *n, int count, size_t rows, int bm) {
     GemmPlan p{};
     p.kbs = (int)(k / 128);
     p.bm = bm;
     p.mtiles = (int)((rows + p.bm - 1) / p.bm);
     GemmSegment direct[kGemvMaxTargets], split[kGemvMaxTargets];
-    int nd = 0, ns = 0, nbs = 0;
-    bool many = count > 1;  // every matrix has a tile per CU and more: they share full rounds and one tail
-    for (int i = 0; i < count; ++i) {
-        nbs += (int)(n[i] / 128);
-        many = many && (int)(n[i] / 128) * p.mtiles > kGemmTargetWgs;
-    }
-    if (many) {
-        gemm_add(p, direct, nd, split, ns, 0, nbs, tails);
-    } else {  // each matrix as exl3_hip_mul_mat would split it: the same bits
-        for (int i = 0, nb0 = 0; i < count; ++i) {
-            gemm_add(p, direct, nd, split, ns, nb0, (int)(n[i] / 128), tails);
-            nb0 += (int)(n[i] / 128);
-        }
+    int nd = 0, ns = 0;
+    for (int i = 0, nb0 = 0; i < count; ++i) {
+        GemmSegment g{};
+        g.nb0 = nb0;
+        g.tiles = (int)(n[i] / 128) * p.mtiles;
+        g.splits = gemm_splits(p.kbs, g.tiles, p.bm);
+        g.kq = p.kbs / g.splits;
+        g.kr = p.kbs % g.splits;
+        if (g.splits == 1) direct[nd++] = g;
+        else split[ns++] = g;
+        nb0 += (int)(n[i] / 128);
     }
     if (p.bm < 128 && nd) {  // the 32/64-row tiles need a split
-        if (count == 1) return gemm_plan_bm(k, n, count, rows, 128, tails);
+        if (count == 1) return gemm_plan_bm(k, n, count, rows, 128);
         return p;  // ok stays false
     }
-    if (nd + ns > kGemmMaxSegments || (p.bm == 128 && nd && ns)) return p;  // (two different kernels)
+    if (p.bm == 128 && nd && ns) return p;  // (two different kernels)
     int begin = 0, units = 0;
     size_t blocks = 0;
     for (int i = 0; i < nd + ns; ++i) {  // whole tiles first, they run longest
@@ -767,11 +737,9 @@ static GemmPlan gemm_plan_bm(size_t k, const size_t *n, int count, size_t rows, 
     return p;
 }
 
-GemmPlan gemm_plan(size_t k, size_t n, size_t rows, bool tails) {
-    return gemm_plan_bm(k, &n, 1, rows, gemm_tile_rows(rows), tails);
-}
+GemmPlan gemm_plan(size_t k, size_t n, size_t rows) { return gemm_plan_bm(k, &n, 1, rows, gemm_tile_rows(rows)); }
 GemmPlan gemm_plan_group(size_t k, const size_t *n, int count, size_t rows) {
-    return gemm_plan_bm(k, n, count, rows, gemm_tile_rows(rows), true);
+    return gemm_plan_bm(k, n, count, rows, gemm_tile_rows(rows));
 }
 
 // one tile class: kernel <RB, W> (NSG scheduling groups per k-step, XD activation
@@ -791,12 +759,10 @@ static void launch_gemm_tiles(const GemvTargets &tg, const uint16_t *xh, size_t 
         // SB splits' loads in flight per batch: one batch for up to 16 splits (the
         // 32-row tiles' 16: -0.4 to -0.6 us per call against two batches of 8)
         const dim3 units((unsigned)p.reduce_units);
-        GemmGrid gg = p.grid;
-        const bool one = tg.count == 1;  // at most one segment without a split before it
-        if (one) gg.seg[0] = gg.seg[gg.count - 1];
+        const bool one = tg.count == 1;
         auto reduce = [&](auto sb, auto is_one) {
             gemm_reduce_kernel<RB, WR, decltype(sb)::value, decltype(is_one)::value>
-                <<<units, dim3(256), 0, stream>>>(tg, gg, K, part, exps, y_f16, (int)rows);
+                <<<units, dim3(256), 0, stream>>>(tg, p.grid, K, part, exps, y_f16, (int)rows);
         };
         typedef std::integral_constant<int, 16> S16;
         typedef std::integral_constant<int, 8> S8;

@@ -87,18 +87,17 @@ struct GemvPlan {
     size_t partials_off, exchange_bytes, dummy_off, xpre_off, bytes;
     bool fits;  // the partials fit the exchange (else the call runs as a GEMM)
 };
-// One run of the GEMM's workgroups: the tiles tile0 .. tile0 + tiles - 1, tile t being
-// column group nb0 + t / mtiles (numbered over all targets) and m-tile t % mtiles, each
-// in `splits` k splits (split s has kq + (s < kr) records).
+// The GEMM's workgroups of one matrix: its tiles, tile t being column group nb0 + t /
+// mtiles (numbered over all targets) and m-tile t % mtiles, each in `splits` k splits
+// (split s has kq + (s < kr) records).
 struct GemmSegment {
     int begin;           // first workgroup id, a multiple of 8
-    int nb0, tile0, tiles, splits, kq, kr;
+    int nb0, tiles, splits, kq, kr;
     unsigned part0;      // first (tile, split) partial block, when split
     int unit0;           // first workgroup of the reduction, when split
 };
-constexpr int kGemmMaxSegments = 4;
 struct GemmGrid {
-    GemmSegment seg[kGemmMaxSegments];  // those without a split first
+    GemmSegment seg[kGemvMaxTargets];  // those without a split first
     int count, mtiles, kbs;
 };
 struct GemmPlan {
@@ -115,11 +114,9 @@ bool gemv_serves(size_t k, size_t n, size_t rows);
 // the GEMV for one matrix: up to kGemvSingleMaxRows rows, and at 15..16 rows where
 // a workgroup preps at most kGemvSinglePrepBlocks (record, row) blocks
 bool gemv_serves_single(size_t k, size_t n, size_t rows);
-// tails: the last round's tiles may be split where more tiles than CUs remain whole;
-// without, the plan (and its workspace) splits all tiles or none
-GemmPlan gemm_plan(size_t k, size_t n, size_t rows, bool tails);
-// the matrices of a grouped call in one launch: below a tile per CU each split as
-// gemm_plan splits it alone, above all together
+GemmPlan gemm_plan(size_t k, size_t n, size_t rows);
+// the matrices of a grouped call in one launch, each with the tiles and splits that
+// gemm_plan gives it alone (the same bits)
 GemmPlan gemm_plan_group(size_t k, const size_t *n, int count, size_t rows);
 int gemm_tile_rows(size_t rows);
 
@@ -150,9 +147,5 @@ hipError_t launch_pack_records(const uint16_t *packed, const uint16_t *su, const
                                size_t n, void *records, hipStream_t stream);
 hipError_t launch_validate(const void *records, size_t nrecords, int bits, int *result, hipStream_t stream);
 hipError_t launch_zero(void *ptr, size_t bytes, hipStream_t stream);
-
-// The least workspace exl3_hip_mul_mat takes (exl3_api.cpp): plans without split tails.
-// exl3_hip_mul_mat_workspace_bytes reports what the fastest plans need.
-size_t mul_mat_least_workspace(size_t k, size_t n, size_t rows);
 
 }  // namespace exl3k

@@ -48,7 +48,7 @@ extern "C" exl3_status exl3_hip_mul_mat_noalloc(const void *records, unsigned bi
                                                 hipStream_t stream) {
     if (!exl3_hip_supports_mul_mat(bits, codebook, k, n, rows, xt, yt)) return EXL3_INVAL_PARAMS;
     // workspaces beyond the array are refused before anything is enqueued
-    if (exl3k::mul_mat_least_workspace(k, n, rows) > kNoallocScratchBytes) return EXL3_WORKSPACE_TOO_SMALL;
+    if (exl3_hip_mul_mat_workspace_bytes(k, n, rows) > kNoallocScratchBytes) return EXL3_WORKSPACE_TOO_SMALL;
     void *ws = nullptr;
     const exl3_status st = scratch_of_current_device(stream, &ws);
     if (st != EXL3_OK) return st;
