@@ -96,6 +96,20 @@ def test_gemv_rows_match_one_row_bitwise(amd, k, n, bits):
         assert not bad
 
 
+@pytest.mark.parametrize("k,n", [(8192, 6144), (8192, 5120), (11008, 4096), (4096, 6144), (8192, 3072)])
+def test_gemv_rows_match_one_row_around_one_workgroup_per_cu(amd, k, n):
+    """The same where one workgroup per CU is in question: three shapes whose share of k would not fit
+    a workgroup at some of 1..14 rows, two where it fits at all of them."""
+    rd = dev(make_layer(432, k, n, 2))
+    x = synth.activations(433, 14, k)
+    ones = np.concatenate([run(amd, rd, 2, k, n, x[r:r + 1]) for r in range(14)])
+    for rows in range(2, 15):
+        y = run(amd, rd, 2, k, n, x[:rows])
+        bad = [r for r in range(rows) if not np.array_equal(y[r], ones[r])]
+        print(f"  k={k} n={n} rows={rows}: rows differing from one-row calls {bad}", flush=True)
+        assert not bad
+
+
 @pytest.mark.parametrize("k,n,bits", [(2048, 2048, 6), (2048, 512, 6), (6144, 2048, 3), (14336, 4096, 4)])
 @pytest.mark.parametrize("rows", [15, 16])
 def test_rows_15_16_short_k_on_gemv(amd, oracle, k, n, bits, rows):

@@ -702,11 +702,11 @@ GemvPlan gemv_plan(size_t k, size_t n, size_t rows) {
     s = (p.kbs + (p.kbs + s - 1) / s - 1) / ((p.kbs + s - 1) / s);
     // a workgroup's B fragments must fit its LDS budget and a wave prepares at
     // most kGemvPrepMax (kb, row) blocks; one kb per workgroup always fits
-    auto serves = [&](int splits) {
+    auto serves = [&](int splits, size_t r) {
         const size_t nkb = ((size_t)p.kbs + splits - 1) / splits;
-        const bool ok_lds = nkb * gemv_frag_bytes_per_kb(rows) <= (rows > 8 ? kGemvFragLds16 : kGemvFragLds);
+        const bool ok_lds = nkb * gemv_frag_bytes_per_kb(r) <= (r > 8 ? kGemvFragLds16 : kGemvFragLds);
         // above 16 rows the activations are prepared once per call (gemv_xprep_kernel)
-        const bool ok_prep = rows > 16 || (nkb * rows + kGemvWaves - 1) / kGemvWaves <= (size_t)kGemvPrepMax;
+        const bool ok_prep = r > 16 || (nkb * r + kGemvWaves - 1) / kGemvWaves <= (size_t)kGemvPrepMax;
         return ok_lds && ok_prep;
     };
     // between one and two workgroups per CU some CUs run two in turn and others idle: one
@@ -714,12 +714,14 @@ GemvPlan gemv_plan(size_t k, size_t n, size_t rows) {
     // of k = 4096, 8 -> 5 splits: rows 1 10.6 -> 9.4 us, rows 8 12.3 -> 10.7; k = 8192,
     // n = 3072, 16 -> 10: 9.2 -> 8.9 and 11.3 -> 10.9).  With as many records either way
     // neither is better throughout (k = 14336, n = 4096 16 splits 13.1, 8 splits 14.4;
-    // 2 x 14336 of k = 4096 2 splits 23.5, none 22.1)
+    // 2 x 14336 of k = 4096 2 splits 23.5, none 22.1).  Only where it serves every row count
+    // up to kGemvSingleMaxRows (the most rows of each mode decide, at most 9 records), so that
+    // the split of k, and with it a row's bits, stays the same for all of them
     const int one = 256 / p.nbs, rounds = (p.nbs * s + 255) / 256;
-    if (rows <= (size_t)kGemvSingleMaxRows && rounds > 1 && one >= 1 && serves(one) &&
-        (p.kbs + one - 1) / one < rounds * ((p.kbs + s - 1) / s))
+    if (rows <= (size_t)kGemvSingleMaxRows && rounds > 1 && one >= 1 && serves(one, 8) &&
+        serves(one, kGemvSingleMaxRows) && (p.kbs + one - 1) / one < rounds * ((p.kbs + s - 1) / s))
         s = one;
-    while (!serves(s) && s < p.kbs) ++s;
+    while (!serves(s, rows) && s < p.kbs) ++s;
     p.splits = s;
     p.nkw = (p.kbs + s - 1) / s;
     p.partials_off = 0;  // the exchange
