@@ -158,20 +158,26 @@ struct GemmColumn {
 };
 // (Static indexes and selects here and below: the kernel arguments then arrive in a few
 // wide scalar loads, all at once; loads at computed indexes, one behind the other, cost
-// 1.3 us per call at M = 512.)
+// 1.3 us per call at M = 512.  The other targets' arguments are read and selected from
+// behind a branch only, which one target does not take: read by every call they cost a
+// single matrix 0.2 to 0.4 us (k = 2048, n = 512, 6 bits, 37 rows 11.2 -> 11.0 us, 512 rows 18.8 -> 18.5).  The
+// empty asm keeps the compiler from turning the branch into selects.)
 template <bool ONE>
 __device__ __forceinline__ GemmColumn gemm_column(const GemvTargets &tg, int nb, size_t colgroup_bytes) {
     GemmColumn c{tg.records[0], tg.y[0], tg.res[0], tg.y_stride[0], tg.res_stride[0], 0, nb};
+    if (!ONE && tg.count > 1) {
+        asm volatile("");
 #pragma unroll
-    for (int i = 1; i < (ONE ? 1 : kGemvMaxTargets); ++i) {
-        const bool in = i < tg.count && nb >= tg.nb_end[i - 1];
-        c.colgroup = in ? tg.records[i] : c.colgroup;
-        c.y = in ? tg.y[i] : c.y;
-        c.res = in ? tg.res[i] : c.res;
-        c.y_stride = in ? tg.y_stride[i] : c.y_stride;
-        c.res_stride = in ? tg.res_stride[i] : c.res_stride;
-        c.target = in ? i : c.target;
-        c.nb = in ? nb - tg.nb_end[i - 1] : c.nb;
+        for (int i = 1; i < kGemvMaxTargets; ++i) {
+            const bool in = i < tg.count && nb >= tg.nb_end[i - 1];
+            c.colgroup = in ? tg.records[i] : c.colgroup;
+            c.y = in ? tg.y[i] : c.y;
+            c.res = in ? tg.res[i] : c.res;
+            c.y_stride = in ? tg.y_stride[i] : c.y_stride;
+            c.res_stride = in ? tg.res_stride[i] : c.res_stride;
+            c.target = in ? i : c.target;
+            c.nb = in ? nb - tg.nb_end[i - 1] : c.nb;
+        }
     }
     c.colgroup += (size_t)c.nb * colgroup_bytes;
     return c;
@@ -181,18 +187,21 @@ __device__ __forceinline__ GemmColumn gemm_column(const GemvTargets &tg, int nb,
 template <bool UNIT>
 __device__ __forceinline__ GemmSegment gemm_segment(const GemmGrid &gg, int id) {
     GemmSegment s = gg.seg[0];
+    if (gg.count > 1) {
+        asm volatile("");
 #pragma unroll
-    for (int i = 1; i < kGemvMaxTargets; ++i) {
-        const GemmSegment &c = gg.seg[i];
-        const bool in = i < gg.count && id >= (UNIT ? c.unit0 : c.begin);
-        s.begin = in ? c.begin : s.begin;
-        s.nb0 = in ? c.nb0 : s.nb0;
-        s.tiles = in ? c.tiles : s.tiles;
-        s.splits = in ? c.splits : s.splits;
-        s.kq = in ? c.kq : s.kq;
-        s.kr = in ? c.kr : s.kr;
-        s.part0 = in ? c.part0 : s.part0;
-        s.unit0 = in ? c.unit0 : s.unit0;
+        for (int i = 1; i < kGemvMaxTargets; ++i) {
+            const GemmSegment &c = gg.seg[i];
+            const bool in = i < gg.count && id >= (UNIT ? c.unit0 : c.begin);
+            s.begin = in ? c.begin : s.begin;
+            s.nb0 = in ? c.nb0 : s.nb0;
+            s.tiles = in ? c.tiles : s.tiles;
+            s.splits = in ? c.splits : s.splits;
+            s.kq = in ? c.kq : s.kq;
+            s.kr = in ? c.kr : s.kr;
+            s.part0 = in ? c.part0 : s.part0;
+            s.unit0 = in ? c.unit0 : s.unit0;
+        }
     }
     return s;
 }
