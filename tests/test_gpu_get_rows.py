@@ -91,9 +91,8 @@ def test_get_rows_strides_bad_ids_and_empty(amd, oracle):
 @pytest.mark.parametrize("count", [2, 9, 511, 512, 513, 1100])
 @pytest.mark.parametrize("bits,cb,k,n", [(6, 2, 256, 384), (3, 0, 128, 1280), (5, 1, 128, 640)])
 def test_get_rows_shared_column_groups(amd, oracle, count, bits, cb, k, n):
-    """Many ids per column group (more than one workgroup serves at once, windows of ids cut
-    between them), repeated and out-of-range ids among them, every column of the group, and a
-    column group of equal weights (exact zeros): every row as the oracle gives it."""
+    """Many ids per column group, repeated and out-of-range ids among them, every column of a group,
+    and a column group of equal weights (exact zeros): every row as the oracle gives it."""
     rng = np.random.default_rng(count * 8 + bits)
     p = synth.packed_tiles(70 + bits, k, n, bits)
     p.reshape(k // 16, n // 16, -1)[:, 8:16] = 0
@@ -107,5 +106,25 @@ def test_get_rows_shared_column_groups(amd, oracle, count, bits, cb, k, n):
     got = amd.get_rows(dev(rec_h), bits, k, n, ids_tensor(ids), codebook=cb).cpu().numpy()
     ok = (ids >= 0) & (ids < n)
     want = oracle.get_rows(rec_h, bits, cb, k, n, ids[ok])
+    assert np.array_equal(got[ok].view(np.uint32), want.view(np.uint32))
+    assert np.all(got[~ok].view(np.uint32) == 0x7FC00000)
+
+
+@pytest.mark.parametrize("k,n,bits,count", [(128, 256, 4, 65535), (128, 384, 3, 65536), (256, 256, 8, 66000)])
+def test_get_rows_many_ids(amd, oracle, k, n, bits, count):
+    """65,535 ids fill the grid's second dimension, more reach its third.  Repeated ids everywhere and
+    ids out of range, on both sides of 65,535 among them: every row as the oracle gives it."""
+    rng = np.random.default_rng(count + bits)
+    p = synth.packed_tiles(90 + bits, k, n, bits)
+    su, sv = synth.layer_scales(90 + bits, k, n)
+    rec_h = synth.pack_records(p, su, sv, bits).view(np.uint8)
+    ids = rng.integers(0, n, count).astype(np.int32)
+    bad = np.unique(np.concatenate([rng.integers(0, count, count // 50), [0, 65533, count - 1],
+                                    [65536, 65537] if count > 65537 else []])).astype(np.int64)
+    ids[bad] = np.where(bad % 2 == 0, n, -1)
+    print(f"  get_rows many {k}x{n} bits={bits} count={count}", flush=True)
+    got = amd.get_rows(dev(rec_h), bits, k, n, ids_tensor(ids)).cpu().numpy()
+    ok = (ids >= 0) & (ids < n)
+    want = oracle.get_rows(rec_h, bits, 2, k, n, np.arange(n, dtype=np.int32))[ids[ok]]
     assert np.array_equal(got[ok].view(np.uint32), want.view(np.uint32))
     assert np.all(got[~ok].view(np.uint32) == 0x7FC00000)

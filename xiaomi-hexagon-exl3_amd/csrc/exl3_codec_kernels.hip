@@ -411,13 +411,8 @@ hipError_t launch_reconstruct(const void *src, int rl, const uint16_t *su, const
 // GET_ROWS on records (src/exl3-ggml.cpp:19-49): out[r][128 kb .. +127] = column
 // c = ids[r] % 128 of the original-basis reconstruct of record (ids[r] / 128, kb) as
 // a 128x128 matrix, fp16-rounded (then widened for F32 output).  Workgroup (r, kb)
-// decodes that record once, wave tr its tile row tr (decode_tile_row), and serves up
-// to kGetRowsShare ids with it: the ids of r's window (kGetRowsWindow ids from a
-// multiple of it) with the same column group are numbered in order, the workgroup
-// whose own number is a multiple of kGetRowsShare takes its and the next ones, the
-// others end.  512 ids of a 151,936-row vocabulary lie in about 416 column groups, a
-// prompt's repeated tokens in fewer.
-// Per id the H128 over n is restricted to the operations output c depends on (the
+// decodes that record, wave tr its tile row tr (decode_tile_row).
+// The H128 over n is restricted to the operations output c depends on (the
 // same butterflies in the same order: bit-exact): a stage of stride 2^s keeps
 // lo + hi, or lo - hi where bit s of c is set.  Strides 1, 2, 4 and 16 pair lanes, and
 // each halves a lane's rows: of two rows A and B the lower lane keeps A's result and
@@ -428,15 +423,15 @@ hipError_t launch_reconstruct(const void *src, int rl, const uint16_t *su, const
 // fma(v, +-scale, +0), as in reconstruct_kernel.
 // An id outside [0, n) writes a NaN row and sets *bad_ids (if given) to 1.
 // Bound: VALU (about 7 per weight, four of them the decode, and 150 per wave around
-// it) and the chain ids -> words -> counting, hidden only by the four workgroups of a
-// CU.  512 ids of a k = 2048, n = 151,936, 6-bit table: 80.5 -> 39.1 us, against a
-// decode into LDS per id and one thread per row for the H128 over n.  With the ids
-// fastest in the grid instead of the records 44.3 us; without the shared decode about
-// a fifth more records; two records per workgroup 48.4 us (80 VGPRs: three workgroups
-// per CU).
+// it) and the chain id -> words -> column, hidden only by the four workgroups of a
+// CU.  512 ids of a k = 2048, n = 151,936, 6-bit table: 79 -> 32.5 us, against a
+// decode into LDS and one thread per row for the H128 over n.  One decode for up to
+// eight ids of a column group, counted among 512 ids, is slower: 40.4 us there (5 more
+// with the ids fastest in the grid instead of the records), and the ids of a run wait for
+// each other (20 equal ids of a 1,024-wide table, 4 bits, 7.1 us against 3.0; 2,048 of a
+// 512-wide one, 3 bits, 115 against 30).  It gains 3 to 5 % only where nearly every
+// group has eight ids and more (2,048 ids in 64 groups, k = 4096, 3 bits, 205 against 212).
 constexpr int kGetRowsThreads = 512;
-constexpr int kGetRowsWindow = kGetRowsThreads;  // one id per thread
-constexpr int kGetRowsShare = 8;                 // ids per decoded record: one per wave at the end
 
 // One lane-pair stage of two values A, B (rows kept by the lower and the upper lane
 // of the pair over block bit S): hi' + al own.  up is all ones on the upper lane: the
@@ -455,21 +450,15 @@ __global__ __launch_bounds__(kGetRowsThreads) __attribute__((amdgpu_waves_per_eu
     const uint8_t *__restrict__ records, size_t k, size_t n, const int32_t *__restrict__ ids, size_t ids_stride,
     size_t count, void *__restrict__ out, int out_f16, size_t out_stride, int *__restrict__ bad_ids) {
     constexpr float kScale = 0.08838834764831844055f;
-    constexpr int W = kGetRowsThreads / 64;
-    __shared__ float colv[kGetRowsShare][128];
-    __shared__ int matches[W];
-    __shared__ int member_row[kGetRowsShare], member_col[kGetRowsShare];
+    __shared__ float colv[128];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // records fastest: the workgroups in flight read whole column groups, each one contiguous
     const size_t r = blockIdx.y + (size_t)gridDim.y * blockIdx.z, kb = blockIdx.x;
     if (r >= count) return;
-    const size_t w0 = r - r % kGetRowsWindow;  // r's window of ids, one per thread
-    const int self = (int)(r - w0);
     const int32_t id = ids[r * ids_stride];
-    const int32_t other = ids[(w0 + tid < count ? w0 + tid : r) * ids_stride];
+    const size_t o = r * out_stride + kb * 128;
     if (id < 0 || (size_t)id >= n) {
-        const size_t o = r * out_stride + kb * 128;
         if (tid < 128) {
             if (out_f16) ((uint16_t *)out)[o + tid] = 0x7e00u;
             else ((uint32_t *)out)[o + tid] = 0x7fc00000u;
@@ -478,105 +467,66 @@ __global__ __launch_bounds__(kGetRowsThreads) __attribute__((amdgpu_waves_per_eu
         return;
     }
     const size_t nb = (size_t)id >> 7;
-    // the record's loads go out before the ids are counted
+    const int c = id & 127;
     uint32_t w[K];
     load_tile_row<K>(records, 1, k, n, kb * 8 + wave, nb * 8, lane, w);
     const uint8_t *rec = records + (nb * (k >> 7) + kb) * group_bytes(K);
     const uint16_t *su = (const uint16_t *)(rec + 2048 * K);
-    const uint16_t sua = su[lane], sub = su[lane + 64];
-    // the ids of the window in this column group, numbered in order
-    const bool match = w0 + tid < count && other >= 0 && (size_t)other < n && (size_t)(other >> 7) == nb;
-    const uint64_t ball = __builtin_amdgcn_ballot_w64(match);
-    const int below = __builtin_popcountll(ball & (((uint64_t)1 << lane) - 1));
-    if (lane == 0) matches[wave] = __builtin_popcountll(ball);
-    if (tid == self) member_row[0] = below;  // r's number within its wave, until the next barrier
-    __syncthreads();
-    int first = member_row[0], total = 0, before = 0;  // r's number, all matches, those of the waves before this one
-#pragma unroll
-    for (int i = 0; i < W; ++i) {
-        const int m = __builtin_amdgcn_readfirstlane(matches[i]);
-        total += m;
-        if (i < (self >> 6)) first += m;
-        if (i < wave) before += m;
-    }
-    first = __builtin_amdgcn_readfirstlane(first);
-    if (first % kGetRowsShare) return;  // uniform: another workgroup serves r
-    const int nids = total - first < kGetRowsShare ? total - first : kGetRowsShare;
+    const uint16_t sua = su[lane], sub = su[lane + 64];  // for the end, behind the words
+    const uint16_t svc = ((const uint16_t *)(rec + 2048 * K + 256))[c];
     u4 frag[4];
     decode_tile_row<K, CB>(w, lane, frag);
-    __syncthreads();  // member_row[0] has been read
-    const int at = before + below - first;
-    if (match && at >= 0 && at < kGetRowsShare) {
-        member_row[at] = tid;
-        member_col[at] = other & 127;
-    }
-    __syncthreads();
     const int b = h128_lane_block(lane & 15);
     uint32_t up1 = (b & 1) ? ~0u : 0u, up2 = (b & 2) ? ~0u : 0u, up4 = (b & 4) ? ~0u : 0u, up8 = (b & 8) ? ~0u : 0u;
     asm("" : "+v"(up1), "+v"(up2), "+v"(up4), "+v"(up8));  // masks, not conditions
-    // this lane's row of the tile row: block bits 2, 1, 0 and the half of its row pair (bit 3)
-    const int row = 16 * wave + (up4 & 8) + (up2 & 4) + (up1 & 2) + (up8 & 1);
-    const float svc = half_bits_to_float(((const uint16_t *)(rec + 2048 * K + 256))[wave < nids ? member_col[wave] : 0]);
-    // the operands of stride 1, on packed row pairs: the same for every id
-    uint32_t own[4][2], got[4][2];
+    float al[7];
+#pragma unroll
+    for (int s = 0; s < 7; ++s) al[s] = (c >> s) & 1 ? -1.f : 1.f;
+    float t[4][2][2];  // stride 1, on packed row pairs: [f][row pair][row], rows 8 (f % 2) + 4 pair + 2 b0 + row
 #pragma unroll
     for (int f = 0; f < 4; ++f)
 #pragma unroll
         for (int vp = 0; vp < 2; ++vp) {
             const uint32_t lo = vp ? frag[f].z : frag[f].x, hi = vp ? frag[f].w : frag[f].y;
-            own[f][vp] = pick(up1, lo, hi);
-            got[f][vp] = (uint32_t)__builtin_amdgcn_mov_dpp((int)pick(up1, hi, lo), 0xB1, 0xF, 0xF, false);
+            const uint32_t own = pick(up1, lo, hi);
+            const uint32_t got = (uint32_t)__builtin_amdgcn_mov_dpp((int)pick(up1, hi, lo), 0xB1, 0xF, 0xF, false);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                t[f][vp][h] = __builtin_fmaf(half_bits_to_float((uint16_t)(own >> (16 * h))), al[0],
+                                             half_bits_to_float((uint16_t)(got >> (16 * h))));
         }
-#pragma unroll 1
-    for (int q = 0; q < nids; ++q) {
-        const int c = __builtin_amdgcn_readfirstlane(member_col[q]);
-        float al[7];
+    float e[4][2];  // stride 2: rows 8 (f % 2) + 4 b1 + 2 b0 + row
 #pragma unroll
-        for (int s = 0; s < 7; ++s) al[s] = (c >> s) & 1 ? -1.f : 1.f;
+    for (int f = 0; f < 4; ++f)
 #pragma unroll
-        for (int f = 0; f < 4; ++f)  // kept packed: hoisted out of the loop as 32 binary32 values they would spill
-            asm volatile("" : "+v"(own[f][0]), "+v"(own[f][1]), "+v"(got[f][0]), "+v"(got[f][1]));
-        float t[4][2][2];  // [f][row pair][row]: rows 8 (f % 2) + 4 pair + 2 b0 + row
+        for (int h = 0; h < 2; ++h) e[f][h] = fold_pair<2>(t[f][0][h], t[f][1][h], up2, al[1]);
+    float g[2][2];  // stride 4: rows 8 b2 + 4 b1 + 2 b0 + row, column half f / 2
 #pragma unroll
-        for (int f = 0; f < 4; ++f)
+    for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
-            for (int vp = 0; vp < 2; ++vp)  // stride 1
+        for (int h = 0; h < 2; ++h) g[ch][h] = fold_pair<4>(e[2 * ch][h], e[2 * ch + 1][h], up4, al[2]);
+    float a[2];  // stride 8: the column halves
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    t[f][vp][h] = __builtin_fmaf(half_bits_to_float((uint16_t)(own[f][vp] >> (16 * h))), al[0],
-                                                 half_bits_to_float((uint16_t)(got[f][vp] >> (16 * h))));
-        float e[4][2];  // stride 2: rows 8 (f % 2) + 4 b1 + 2 b0 + row
-#pragma unroll
-        for (int f = 0; f < 4; ++f)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) e[f][h] = fold_pair<2>(t[f][0][h], t[f][1][h], up2, al[1]);
-        float g[2][2];  // stride 4: rows 8 b2 + 4 b1 + 2 b0 + row, column half f / 2
-#pragma unroll
-        for (int ch = 0; ch < 2; ++ch)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) g[ch][h] = fold_pair<4>(e[2 * ch][h], e[2 * ch + 1][h], up4, al[2]);
-        float a[2];  // stride 8: the column halves
-#pragma unroll
-        for (int h = 0; h < 2; ++h) a[h] = __builtin_fmaf(g[1][h], al[3], g[0][h]);
-        float z = fold_pair<8>(a[0], a[1], up8, al[4]);  // stride 16: row pair split over b3
-        {  // strides 32, 64: every lane of the four 16-lane rows ends with the sum
-            const auto s32 = __builtin_amdgcn_permlane16_swap(__float_as_int(z), __float_as_int(z), false, false);
-            z = __builtin_fmaf(__int_as_float(s32[1]), al[5], __int_as_float(s32[0]));
-            const auto s64 = __builtin_amdgcn_permlane32_swap(__float_as_int(z), __float_as_int(z), false, false);
-            z = __builtin_fmaf(__int_as_float(s64[1]), al[6], __int_as_float(s64[0]));
-        }
-        // the lower lane of a pair holds own +- hi negated where the stage subtracts
-        const uint32_t neg = ((c & 1) ? ~up1 : 0u) ^ ((c & 2) ? ~up2 : 0u) ^ ((c & 4) ? ~up4 : 0u) ^ ((c & 16) ? ~up8 : 0u);
-        const float scale = __uint_as_float(__float_as_uint(kScale) ^ (neg & 0x80000000u));
-        if (lane < 16) colv[q][row] = __builtin_fmaf(z, scale, 0.f);
+    for (int h = 0; h < 2; ++h) a[h] = __builtin_fmaf(g[1][h], al[3], g[0][h]);
+    float z = fold_pair<8>(a[0], a[1], up8, al[4]);  // stride 16: row pair split over b3
+    {  // strides 32, 64: every lane of the four 16-lane rows ends with the sum
+        const auto s32 = __builtin_amdgcn_permlane16_swap(__float_as_int(z), __float_as_int(z), false, false);
+        z = __builtin_fmaf(__int_as_float(s32[1]), al[5], __int_as_float(s32[0]));
+        const auto s64 = __builtin_amdgcn_permlane32_swap(__float_as_int(z), __float_as_int(z), false, false);
+        z = __builtin_fmaf(__int_as_float(s64[1]), al[6], __int_as_float(s64[0]));
     }
+    // the lower lane of a pair holds own +- hi negated where the stage subtracts
+    const uint32_t neg = ((c & 1) ? ~up1 : 0u) ^ ((c & 2) ? ~up2 : 0u) ^ ((c & 4) ? ~up4 : 0u) ^ ((c & 16) ? ~up8 : 0u);
+    const float scale = __uint_as_float(__float_as_uint(kScale) ^ (neg & 0x80000000u));
+    // this lane's row of the tile row: block bits 2, 1, 0 and the half of its row pair (bit 3)
+    const int row = 16 * wave + (up4 & 8) + (up2 & 4) + (up1 & 2) + (up8 & 1);
+    if (lane < 16) colv[row] = __builtin_fmaf(z, scale, 0.f);
     __syncthreads();
-    if (wave < nids) {
-        float e0 = colv[wave][lane], e1 = colv[wave][lane + 64];
+    if (wave == 0) {
+        float e0 = colv[lane], e1 = colv[lane + 64];
         h128_wave(e0, e1, lane);
-        const uint16_t h0 = float_to_half_bits(mul_rn_f32(mul_rn_f32(e0, half_bits_to_float(sua)), svc));
-        const uint16_t h1 = float_to_half_bits(mul_rn_f32(mul_rn_f32(e1, half_bits_to_float(sub)), svc));
-        const size_t o = (w0 + member_row[wave]) * out_stride + kb * 128;
+        const uint16_t h0 = float_to_half_bits(mul_rn_f32(mul_rn_f32(e0, half_bits_to_float(sua)), half_bits_to_float(svc)));
+        const uint16_t h1 = float_to_half_bits(mul_rn_f32(mul_rn_f32(e1, half_bits_to_float(sub)), half_bits_to_float(svc)));
         if (out_f16) {
             ((uint16_t *)out)[o + lane] = h0;
             ((uint16_t *)out)[o + lane + 64] = h1;
