@@ -218,8 +218,8 @@ def test_nd_entries_and_group_sizing_host_checks():
                                   ctypes.byref(T(a.GGML_F32, [k, 4])), None, None) == 1
     assert L.exl3_hip_get_rows_nd(R, 4, 2, k, n, X, ctypes.byref(T(a.GGML_I32, [0])), Y,
                                   ctypes.byref(T(a.GGML_F32, [k, 0])), None, None) == 0   # no ids: no-op
-    # group sizing: gate/up k = 2048, n = 8192 each, at 513 and 520 rows; the GEMM path runs one
-    # exl3_hip_mul_mat per matrix, whose split partials may exceed the total width's
+    # group sizing: gate/up k = 2048, n = 8192 each, at 513 and 520 rows; the GEMM's activations and
+    # split partials per matrix may exceed the total width's
     for rows in (513, 520, 33, 8):
         g = a.group_workspace_bytes(2048, [8192, 8192], rows)
         assert g >= L.exl3_hip_mul_mat_workspace_bytes(2048, 8192, rows), rows

@@ -336,7 +336,7 @@ def test_group_matches_single_layers(amd, oracle, rows):
     """q/k/v and gate/up of one decoder layer through exl3_hip_mul_mat_group: one GEMV
     launch (rows <= 32; above 16 after one activation pass for all matrices) that serves
     several matrices sharing x; each output within the layer tolerance of the oracle,
-    and above (one call per matrix) equal to mul_mat"""
+    and above (one GEMM launch) equal to mul_mat"""
     import torch
     for k, shapes, bits in [(2048, [2048, 512, 512], 6), (2048, [6144, 6144], 4)]:
         recs = [make_layer(700 + i + bits, k, n, bits) for i, n in enumerate(shapes)]
@@ -355,8 +355,8 @@ def test_group_matches_single_layers(amd, oracle, rows):
 
 @pytest.mark.parametrize("rows", [520, 33])
 def test_group_workspace_of_documented_size(amd, rows):
-    """gate/up (k = 2048, n = 8192 each) at rows where the group runs one exl3_hip_mul_mat
-    per matrix, whose split partials need more than the total width's plan: a caller
+    """gate/up (k = 2048, n = 8192 each) at rows where the group runs one GEMM launch, whose
+    activations and split partials per matrix need more than the total width's plan: a caller
     workspace of exactly exl3_hip_mul_mat_group_workspace_bytes is accepted, and each
     output equals exl3_hip_mul_mat's bit for bit"""
     import torch
@@ -604,6 +604,41 @@ def test_group_gemm_one_launch_equals_single_calls(amd, oracle, rows, shapes):
     ref = oracle.mul_mat(make_layer(1500, k, shapes[0], bits), bits, 2, k, shapes[0],
                          synth.activations(1510 + rows, rows, k))
     assert_layer_close(single[0].cpu().numpy(), ref, what=f"group gemm rows={rows}")
+
+
+def test_group_internal_workspace_under_capture(amd):
+    """A grouped GEMM captured while the internal workspace holds its calls one by one but not their one
+    launch records those calls; the next eager call grows the workspace and runs the one launch.
+    The same bits from both, before and after, and from each matrix alone."""
+    import torch
+    k, bits, rows, ns = 640, 3, 300, [1280, 128]
+    recs = [dev(make_layer(1700 + i, k, n, bits)) for i, n in enumerate(ns)]
+    x = torch.from_numpy(synth.activations(1701, rows, k)).cuda()
+    single = [amd.mul_mat(r, bits, k, n, x) for r, n in zip(recs, ns)]
+    sizes = {n: amd.workspace_bytes(k, n, rows) for n in (*ns, sum(ns))}
+    most = max(sizes, key=sizes.get)
+    assert amd.group_workspace_bytes(k, ns, rows) > sizes[most]
+    both = torch.cat([r.view(torch.uint8).reshape(-1) for r in recs])
+    s = torch.cuda.Stream()  # its internal workspace is new
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        amd.mul_mat({**dict(zip(ns, recs)), sum(ns): both}[most], bits, k, most, x, stream=s)
+    torch.cuda.synchronize()
+    ys = [torch.empty((rows, n), device="cuda") for n in ns]
+    mats = [(r, n, y) for r, n, y in zip(recs, ns, ys)]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        amd.mul_mat_group(mats, bits, k, x, stream=s)
+    for rep in range(3):
+        for y in ys:
+            y.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, want) for y, want in zip(ys, single)), rep
+        with torch.cuda.stream(s):
+            eager = amd.mul_mat_group(list(zip(recs, ns)), bits, k, x, stream=s)
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, want) for y, want in zip(eager, single)), rep
 
 
 @pytest.mark.parametrize("rows,ns", [(260, [33024]), (260, [40960]), (600, [16640]), (260, [33024, 33152]),

@@ -1,5 +1,6 @@
-// exl3_gemm.hip -- the EXL3 layer at rows > 32 on gfx950 (gemm_xprep_kernel,
-// gemm_kernel, gemm_reduce_kernel): H128(x*su) once in fp16 MFMA-fragment order;
+// exl3_gemm.hip -- the EXL3 layer on gfx950 where the GEMV does not serve it: one matrix
+// above 14 rows (16 at short k), grouped calls above 32 and partials beyond the exchange
+// (gemm_xprep_kernel, gemm_kernel, gemm_reduce_kernel): H128(x*su) once in fp16 MFMA-fragment order;
 // a workgroup (k split, column group, m-tile) decodes record kb + 1 into LDS
 // (fp16, swizzled) while v_mfma_f32_32x32x16_f16 runs on record kb, fp32
 // accumulation; split partials are summed in fixed order by the reduce kernel,
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(64) void gemm_xprep_kernel(GemvTargets tg, int bits
     }
 }
 
-// GEMM (rows > 32).  Workgroup (split s, m-tile mt, column group nb) of W waves
+// GEMM.  Workgroup (split s, m-tile mt, column group nb) of W waves
 // (4 or 8): rows [BM mt, +BM) x columns [128 nb, +128), records kb in [kb0, kb1);
 // BM = 32 RB W rows, wave w owning rows 32 RB w .. +32 RB for all 128 columns:
 // RB x 4 accumulator blocks of v_mfma_f32_32x32x16_f16 (one wave per SIMD keeps

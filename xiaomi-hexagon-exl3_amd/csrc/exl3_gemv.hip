@@ -196,7 +196,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) __attribute__((amdgpu_waves_per_eu
     auto group_q = [&](int i) { return part + P * i; };
     auto group_src = [&](int i) -> const uint8_t * {
         const int q = group_q(i);
-        if constexpr (TILES)  // past the last group: the last one again (the dummy region is too small for the pitch)
+        if constexpr (TILES)  // past the last group: the wave's first one again (the dummy region is too small for the pitch)
             return colgroup + (size_t)(8 * kb0 + 4 * (i < ngroups ? q : group_q(0))) * tile_row + lane_off;
         else return i < ngroups ? colgroup + (size_t)(kb0 + (q >> 1)) * GB + (size_t)(q & 1) * 1024 * K + lane_off
                            : dummy + lane_off;

@@ -1,5 +1,5 @@
 // exl3_launch.hpp -- internal launcher interface between the C-ABI (exl3_api.cpp)
-// and the gfx950 kernels (exl3_kernels.hip).  Launchers assume the caller has
+// and the gfx950 kernels (exl3_{gemv,gemm,codec_kernels}.hip).  Launchers assume the caller has
 // validated every argument; they only enqueue work and return hipGetLastError().
 #pragma once
 
