@@ -714,6 +714,9 @@ static GemmPlan gemm_plan_bm(size_t k, const size_t *n, int count, size_t rows, 
         return p;  // ok stays false
     }
     if (p.bm == 128 && nd && ns) return p;  // (two different kernels)
+    if (nd == count) {  // whole tiles only: one segment for all (2 x 14336 of k = 4096 at 4096 rows 0.6 % faster)
+        for (; nd > 1; --nd) direct[0].tiles += direct[nd - 1].tiles;
+    }
     int begin = 0, units = 0;
     size_t blocks = 0;
     for (int i = 0; i < nd + ns; ++i) {  // whole tiles first, they run longest

@@ -87,9 +87,9 @@ struct GemvPlan {
     size_t partials_off, exchange_bytes, dummy_off, xpre_off, bytes;
     bool fits;  // the partials fit the exchange (else the call runs as a GEMM)
 };
-// The GEMM's workgroups of one matrix: its tiles, tile t being column group nb0 + t /
-// mtiles (numbered over all targets) and m-tile t % mtiles, each in `splits` k splits
-// (split s has kq + (s < kr) records).
+// The GEMM's workgroups of one matrix, or of all where none is split over k: its tiles,
+// tile t being column group nb0 + t / mtiles (numbered over all targets) and m-tile t %
+// mtiles, each in `splits` k splits (split s has kq + (s < kr) records).
 struct GemmSegment {
     int begin;           // first workgroup id, a multiple of 8
     int nb0, tiles, splits, kq, kr;
