@@ -114,7 +114,7 @@ exl3_status call_workspace(size_t need, hipStream_t stream, void **workspace, si
 // workspace serves all smaller calls of the same (k, n) in turn (every plan starts
 // with the same exchange region).
 // The last sizes asked for are kept per thread (a pure function of its arguments): a call
-// of 37 rows otherwise plans the smaller row counts again each time (1.7 us of host time).
+// of 37 rows otherwise plans the smaller row counts again each time (0.5 us of host time, 0.8 at 4,096).
 size_t mul_mat_need(size_t k, size_t n, size_t rows) {
     if (!valid_matrix(k, n, 128) || rows < 1 || rows > kMaxRows) return 0;
     struct Kept {
