@@ -545,7 +545,7 @@ def extra_configs(amd, torch, np, synth, stream, args, only_c1=False):
                                "matrices": len(mats), "weights": wsum,
                                "mean_bpw": round(float(sum(k2 * n2 * int(b2) for (k2, n2), b2 in zip(mats, bits_c2)) / wsum), 3),
                                "bytes": c2_bytes, "sweep_ms_one_call_per_matrix": round(ms_each, 3),
-                               "note": "one exl3_hip_decode_batch call (one launch per rate and up to 32 "
+                               "note": "one exl3_hip_decode_batch call (one launch per 32 "
                                        "matrices), each matrix into its own output"}
     del packed, dst, batch, outs
 
